@@ -1160,22 +1160,38 @@ static SkinnyPlan plan_skinny(int M, int N, int K, bool part, bool argmax) {
   p.P = cdiv_i(K, p.kc);
   return p;
 }
-struct MfmaPlan {
-  int P, kchunk, mt, nt;
-};
-constexpr int MFMA_MAX_SPLIT = 8;
+// Tiled MFMA: a CU works through its blocks' tiles at the matrix cores' rate
+// however many it holds, so the launch takes as long as the fullest CU.  Whole
+// rounds of 256 tiles are one block each; the tiles after them (all, when
+// there are fewer) split K so that their blocks fill the CUs evenly.  Cost in
+// K elements of a tile: the fullest CU's share, a fifth more per block when
+// blocks are too few to hide their loads behind each other, and the partials'
+// round trip (60 + 25 per split, about 5 + 2.4 us of the 0.12 us an element
+// takes).  Measured on MI355X, complex, us with one block per tile -> the
+// plan's: 519 x 2304 x 768 (324 tiles) 182 -> 132, with every tile split 145;
+// 855 x 1536 x 512 132 -> 95; 519 x 768 x 3072 (108 tiles) 368 -> 177;
+// 128 x 512 x 2048 246 -> 50; 512 x 512 x 32000 3836 -> 965.
+constexpr int MFMA_CUS = 256;
+constexpr int MFMA_MAX_SPLIT = 16;
+constexpr int MFMA_MAX_PARTS = 1024;  // partial tiles (64 KB each) of a launch
 static MfmaPlan plan_mfma(int M, int N, int K) {
   MfmaPlan p;
-  p.mt = cdiv_i(M, GBM);
-  p.nt = cdiv_i(N, GBN);
-  const int tiles = p.mt * p.nt;
-  int P = 1;
-  // at most MFMA_MAX_SPLIT ways: at config 3, batch 1 (128 prompt rows) FFN
-  // Linear split 32 ways took 199 us, FFN Dense split 8 ways 92 us for the
-  // same flops
-  if (tiles < 512) P = std::min({cdiv_i(512, tiles), std::max(1, K / 64), MFMA_MAX_SPLIT});
-  p.kchunk = cdiv_i(cdiv_i(K, P), GBK) * GBK;
-  p.P = cdiv_i(K, p.kchunk);
+  const int tiles = cdiv_i(M, GBM) * cdiv_i(N, GBN);
+  const int rest = tiles % MFMA_CUS;
+  double best = 0.0;
+  for (int P = 1; P <= MFMA_MAX_SPLIT; ++P) {
+    const int kc = cdiv_i(cdiv_i(K, P), GBK) * GBK;
+    if (P > 1 && (kc < 32 || cdiv_i(K, kc) != P || rest * P > MFMA_MAX_PARTS)) continue;
+    const int load = cdiv_i((long)rest * P, MFMA_CUS);
+    const int held = std::min(3, tiles / MFMA_CUS + load);
+    const double cost = (double)load * kc * (1.0 + 0.2 / std::max(1, held)) + (P > 1 ? 60.0 + 25.0 * P : 0.0);
+    if (P > 1 && cost >= best) continue;
+    best = cost;
+    p.P = P;
+    p.kchunk = kc;
+  }
+  p.whole = p.P > 1 ? tiles - rest : tiles;
+  p.rest = tiles - p.whole;
   return p;
 }
 
@@ -1191,10 +1207,10 @@ int gemm_parts(int M, int N, int K) {
 }
 
 size_t gemm_ws_bytes(int M, int N, int K) {
+  if (M > SKINNY_MAX_M) return plan_mfma(M, N, K).ws_bytes();
   int P;
   if (M <= 8) P = std::max(plan_gemv(M, N, K, false).P, plan_gemv(M, N, K, false, true).P);
-  else if (M <= SKINNY_MAX_M) P = plan_skinny(M, N, K, false, true).P;  // the largest split workspace
-  else P = plan_mfma(M, N, K).P;
+  else P = plan_skinny(M, N, K, false, true).P;  // the largest split workspace
   return P > 1 ? (size_t)P * M * N * sizeof(double2) : 0;
 }
 
@@ -1293,11 +1309,9 @@ int gemm(hipStream_t st, int M, int N, int K, const RowOps& ro, const double2* W
     } else {
       if (ep.mode == EPI_PART) return ERR_ARG;
       const MfmaPlan p = plan_mfma(M, N, K);
-      if (p.P > 1 && (long)p.mt * p.nt >= SYNC_COUNTERS) return ERR_ARG;
-      dim3 grid(p.nt, p.mt, p.P);
-      if (launch_zgemm_mfma(st, grid, ro.x, ro.ldx, W, ldw, M, N, K, p.kchunk, ep, am, (double2*)sy.ws, sy.counters) != OK)
+      if (launch_zgemm_mfma(st, p, ro.x, ro.ldx, ro.real, W, ldw, M, N, K, ep, am, (double2*)sy.ws, sy.counters) != OK)
         return ERR_ARG;
-      tiles = p.nt;
+      tiles = cdiv_i(N, GBN);
     }
   }
   if (am.part_v) MITOK_LAUNCH(k_argmax_finalize, dim3(M), dim3(256), 0, st, am, tiles);

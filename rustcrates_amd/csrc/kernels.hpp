@@ -36,6 +36,7 @@ struct AttnSplit {
 //   -> + bias -> finite check -> GELU -> RoPE -> residual Re(x + r) -> LayerNorm
 struct RowOps {
   const double2* x = nullptr;  // [M][ldx] rows, or partial p at x + p * part_stride
+  bool real = false;           // plain rows whose imaginary parts are zero (a Norm leaves such rows)
   long ldx = 0;
   int npart = 0;  // > 1: x[m][k] = sum over p < npart of the partials, in order
   long part_stride = 0;
@@ -209,10 +210,16 @@ bool attention_prefill(hipStream_t st, const Attn& a);
 // `append` the partials are [q | k | v] of the new token, whose k and v the
 // kernel appends to the cache (kc_w, vc_w).
 // MFMA-tiled GEMM (gemm_mfma.hip) for M > 64: block tile GBM x GBN, K step
-// GBK; grid (N tiles, M tiles, K splits of kchunk).  ERR_ARG for EPI_PART.
-constexpr int GBM = 64, GBN = 64, GBK = 16;
-int launch_zgemm_mfma(hipStream_t st, dim3 grid, const double2* A, long lda, const double2* W, long ldw, int M, int N,
-                      int K, int kchunk, const Epi& ep, const Argmax& am, double2* ws, uint32_t* cnt);
+// GBK; the first `whole` output tiles are one block each, the `rest` P blocks
+// of kchunk of K.  a_real: A's imaginary parts are zero.  ERR_ARG for EPI_PART.
+constexpr int GBM = 64, GBN = 64, GBK = 8;
+struct MfmaPlan {
+  int whole = 0, rest = 0, P = 1, kchunk = 0;
+  long blocks() const { return whole + (long)rest * P; }
+  size_t ws_bytes() const { return P > 1 ? (size_t)rest * P * GBM * GBN * sizeof(double2) : 0; }
+};
+int launch_zgemm_mfma(hipStream_t st, const MfmaPlan& p, const double2* A, long lda, bool a_real, const double2* W,
+                      long ldw, int M, int N, int K, const Epi& ep, const Argmax& am, double2* ws, uint32_t* cnt);
 
 AttnSplit attention_split_plan(const Attn& a);
 size_t attention_split_ws_bytes(int B, int H, int dh, int T_max);

@@ -631,10 +631,11 @@ static Sync sync_of(Net* n) {
   return s;
 }
 
-static RowOps rows_of(const double2* x, long ldx) {
+static RowOps rows_of(const double2* x, long ldx, bool real = false) {
   RowOps r;
   r.x = x;
   r.ldx = ldx;
+  r.real = real;
   return r;
 }
 
@@ -683,6 +684,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
   const uint32_t* lens = sp.lens;
   const int* pos = sp.pos;
   size_t wi = 0;  // next wavelet stage
+  bool real = false;  // the rows in cur have zero imaginary parts: a Norm leaves Re(x) + 0i (norm_layer.rs:64-130)
   double2* cur = n->act0.as<double2>();
   double2* nxt = n->act1.as<double2>();
   if (sp.in) HIP_TRY(hipMemcpyAsync(cur, sp.in, (size_t)rows * n->layers[sp.first]->d_in * sizeof(double2),
@@ -707,6 +709,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         auto* N = (NormLayer*)L;
         layernorm(st, cur, nullptr, nxt, rows, N->d_in, N->eps, N->gamma.as<double2>(), N->beta.as<double2>());
         std::swap(cur, nxt);
+        real = true;
         break;
       }
       case K_SELF_ATTENTION: {
@@ -748,7 +751,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         {
           TimeScope ts(n, S > 1 ? MITOK_TIME_PREFILL_GEMM : MITOK_TIME_LAYER_GEMM, gemm_bytes(rows, 3 * d, d, false),
                        gemm_flops(rows, 3 * d, d));
-          TRY(launch_rc(gemm(st, rows, 3 * d, d, rows_of(cur, d), A->wqkv.as<double2>(), 3 * d, e, nullptr, sy), "qkv"));
+          TRY(launch_rc(gemm(st, rows, 3 * d, d, rows_of(cur, d, real), A->wqkv.as<double2>(), 3 * d, e, nullptr, sy), "qkv"));
         }
         a.kc = e.kc;
         a.vc = e.vc;
@@ -792,6 +795,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
                     A->beta.as<double2>());
         }
         std::swap(cur, nxt);
+        real = true;
         break;
       }
       case K_FEED_FORWARD: {
@@ -813,7 +817,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         {
           TimeScope ts(n, S > 1 ? MITOK_TIME_PREFILL_GEMM : MITOK_TIME_LAYER_GEMM, gemm_bytes(rows, F->hidden, F->d_in, false),
                        gemm_flops(rows, F->hidden, F->d_in));
-          TRY(launch_rc(gemm(st, rows, F->hidden, F->d_in, rows_of(cur, F->d_in), F->w1.as<double2>(), F->hidden, e1,
+          TRY(launch_rc(gemm(st, rows, F->hidden, F->d_in, rows_of(cur, F->d_in, real), F->w1.as<double2>(), F->hidden, e1,
                              nullptr, sy), "ffn1"));
         }
         {
@@ -823,6 +827,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
                              F->w2.as<double2>(), F->d_out, e2, nullptr, sy), "ffn2"));
         }
         std::swap(cur, nxt);
+        real = false;
         break;
       }
       case K_LINEAR: {
@@ -835,9 +840,10 @@ static int enqueue_forward(Net* n, const Spec& sp) {
           e.out = nxt;
           e.ldo = Ln->d_out;
           e.err = err;
-          TRY(launch_rc(gemm(st, rows, Ln->d_out, Ln->d_in, rows_of(cur, Ln->d_in), Ln->w.as<double2>(), Ln->d_out, e,
+          TRY(launch_rc(gemm(st, rows, Ln->d_out, Ln->d_in, rows_of(cur, Ln->d_in, real), Ln->w.as<double2>(), Ln->d_out, e,
                              nullptr, sy), "linear"));
           std::swap(cur, nxt);
+          real = false;
           break;
         }
         const double2* x = cur;
@@ -857,12 +863,12 @@ static int enqueue_forward(Net* n, const Spec& sp) {
           e.hist_re = sp.hist_re;
           e.hist_cnt = sp.hist_cnt;
           TimeScope ts(n, MITOK_TIME_VOCAB, gemm_bytes(M, Ln->d_out, Ln->d_in, true), gemm_flops_re(M, Ln->d_out, Ln->d_in));
-          TRY(launch_rc(gemm(st, M, Ln->d_out, Ln->d_in, rows_of(x, Ln->d_in), Ln->w.as<double2>(), Ln->d_out, e,
+          TRY(launch_rc(gemm(st, M, Ln->d_out, Ln->d_in, rows_of(x, Ln->d_in, real), Ln->w.as<double2>(), Ln->d_out, e,
                              sp.am, sy), "vocab"));
         } else {
           e.mode = EPI_STORE;
           e.out = n->logits_c.as<double2>();
-          TRY(launch_rc(gemm(st, M, Ln->d_out, Ln->d_in, rows_of(x, Ln->d_in), Ln->w.as<double2>(), Ln->d_out, e,
+          TRY(launch_rc(gemm(st, M, Ln->d_out, Ln->d_in, rows_of(x, Ln->d_in, real), Ln->w.as<double2>(), Ln->d_out, e,
                              nullptr, sy), "vocab"));
           if (sp.mode == MODE_STATELESS && !sp.last_row) {  // the layer keeps its input for backward
             n->head_valid = true;
