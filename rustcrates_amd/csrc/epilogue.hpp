@@ -6,6 +6,8 @@
 // resident decode loop (Acc: the access policy, common.hpp).
 #pragma once
 
+#include <type_traits>
+
 #include "rowops.hpp"
 
 namespace mitok {
@@ -22,6 +24,8 @@ __device__ __forceinline__ double apply_epi(const Epi& ep, int M, int N, int m, 
       Acc::st(ep.out + (long)m * ep.ldo + n, v);
       break;
     case EPI_GELU: {
+      if constexpr (std::is_same<Acc, AccPlain>::value)
+        if (ep.pre) ep.pre[(long)m * ep.ldo + n] = v;
       bool nan = false;
       if (ep.row_mask && Acc::c(ep.row_mask + m) == 0) v = make_double2(0.0, 0.0);  // activation.rs:268-284
       else v = gelu_nc(v, &nan);

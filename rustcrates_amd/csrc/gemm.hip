@@ -18,6 +18,7 @@
 #include <algorithm>
 
 #include "epilogue.hpp"
+#include "train.hpp"
 
 namespace mitok {
 
@@ -1214,6 +1215,18 @@ size_t gemm_ws_bytes(int M, int N, int K) {
   return P > 1 ? (size_t)P * M * N * sizeof(double2) : 0;
 }
 
+size_t gemm_tiled_ws_bytes(int M, int N, int K) { return plan_mfma(M, N, K).ws_bytes(); }
+
+int gemm_tiled(hipStream_t st, int M, int N, int K, const GemmOpnd& A, const GemmOpnd& B, const Epi& ep, const Sync& sy,
+               const MfmaBatch& bt) {
+  if (M <= 0 || N <= 0 || bt.n <= 0) return OK;
+  if (K <= 0) return ERR_ARG;
+  MfmaPlan p = plan_mfma(M, N, K);
+  if (bt.n > 1) p = MfmaPlan{cdiv_i(M, GBM) * cdiv_i(N, GBN)};  // the batch fills the chip
+  if (p.ws_bytes() > sy.ws_bytes) return ERR_STATE;
+  return launch_zgemm_mfma(st, p, A, B, M, N, K, ep, Argmax(), (double2*)sy.ws, sy.counters, bt);
+}
+
 // argmax partials: one per row and 16-column tile covers every product shape
 size_t argmax_part_elems(int M, int N) { return (size_t)M * cdiv_i(N, 16); }
 
@@ -1309,8 +1322,8 @@ int gemm(hipStream_t st, int M, int N, int K, const RowOps& ro, const double2* W
     } else {
       if (ep.mode == EPI_PART) return ERR_ARG;
       const MfmaPlan p = plan_mfma(M, N, K);
-      if (launch_zgemm_mfma(st, p, ro.x, ro.ldx, ro.real, W, ldw, M, N, K, ep, am, (double2*)sy.ws, sy.counters) != OK)
-        return ERR_ARG;
+      const GemmOpnd A{ro.x, ro.ldx, ro.real ? OP_RE : 0}, B{W, ldw, 0};
+      if (launch_zgemm_mfma(st, p, A, B, M, N, K, ep, am, (double2*)sy.ws, sy.counters) != OK) return ERR_ARG;
       tiles = cdiv_i(N, GBN);
     }
   }

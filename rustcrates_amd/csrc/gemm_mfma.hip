@@ -9,6 +9,7 @@
 // loads before the first MFMA.  In the VGPR form the loop has no copies.  The
 // flag is kept to this file: the skinny decode products measured slower with it.
 #include "epilogue.hpp"
+#include "train.hpp"
 
 namespace mitok {
 
@@ -45,19 +46,14 @@ namespace mitok {
 // B[k][j] at lane j+16k, D[i][j] at lane j+16*(i%4), element i/4 (unlike the
 // f32 16x16x4 form, consecutive output rows sit in consecutive lane groups).
 //
-// Operands (GemmOpnd): row-major complex as it is, its real part, a
-// row-major array of doubles, or the conjugate transpose of a row-major
-// complex or double array read in place (the products of backward; a
-// materialised transpose cost a pass over memory and a launch each).
+// Operands (GemmOpnd, train.hpp): a row-major complex or double array as it
+// is or transposed, conjugated or not, real or not.  Backward's products read
+// their transposes in place; each materialised one cost a pass over memory
+// and a launch.
 // ===========================================================================
 constexpr int GNT = 512;  // threads
 constexpr int GMT = 2;    // 16-row tiles of a wave
 __device__ const double2 gemm_zero2 = {0.0, 0.0};  // what a load outside the operand reads
-
-// how an operand is read: OP_H conjugate transpose of the stored array,
-// OP_RE its imaginary part is zero (not read into LDS), OP_F64 stored as
-// doubles (implies real)
-constexpr int OP_H = 1, OP_RE = 2, OP_F64 = 4;
 
 // One operand's 64 x 8 tile in LDS.  ALONG_K: the stored array is contiguous
 // along K (A as it is, B transposed): element (i, k) at row i, its k XORed so
@@ -113,13 +109,20 @@ template <int MODE, int AF, int BF>
 __global__ __launch_bounds__(GNT, 6) void k_zgemm_mfma(const void* __restrict__ A, long lda, const void* __restrict__ Bm,
                                                        long ldb, int M, int N, int K, int whole, int splits,
                                                        int kchunk, Epi ep_in, Argmax am, double2* __restrict__ ws,
-                                                       uint32_t* __restrict__ cnt) {
-  using TA = GemmTile<AF, !(AF & OP_H)>;
-  using TB = GemmTile<BF, (BF & OP_H) != 0>;
+                                                       uint32_t* __restrict__ cnt, MfmaBatch bt) {
+  using TA = GemmTile<AF, !(AF & OP_T)>;
+  using TB = GemmTile<BF, (BF & OP_T) != 0>;
   constexpr bool RE = MODE == EPI_RE;  // only the real part is used
   static_assert(!(TA::real && TB::real), "one operand is complex");
   Epi ep = ep_in;
   ep.mode = MODE;
+  if (bt.n > 1) {
+    const long z = blockIdx.y, z0 = z / bt.inner, z1 = z - z0 * bt.inner, c = z0 * bt.c0 + z1 * bt.c1;
+    A = (const typename TA::TG*)A + z0 * bt.a0 + z1 * bt.a1;
+    Bm = (const typename TB::TG*)Bm + z0 * bt.b0 + z1 * bt.b1;
+    if (RE) ep.out_re += c;
+    else ep.out += c;
+  }
   constexpr int STAGE = RE ? GBM * 65 * (int)sizeof(double) : 0;  // Re values of the tile for the fused argmax
   constexpr int TILES = 2 * (TA::BYTES + TB::BYTES);
   __shared__ __align__(16) char lds[TILES > STAGE ? TILES : STAGE];
@@ -169,7 +172,7 @@ __global__ __launch_bounds__(GNT, 6) void k_zgemm_mfma(const void* __restrict__ 
 #pragma unroll
   for (int t = 0; t < GMT; ++t) cr[t] = ci[t] = v4d{0.0, 0.0, 0.0, 0.0};
   // a conjugated operand's imaginary part enters with the other sign
-  constexpr bool NA = (AF & OP_H) != 0, NB = (BF & OP_H) != 0;
+  constexpr bool NA = (AF & OP_CJ) != 0, NB = (BF & OP_CJ) != 0;
   auto mma = [&](int f) {
 #pragma unroll
     for (int t = 0; t < GMT; ++t) {
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(GNT, 6) void k_zgemm_mfma(const void* __restrict__ 
     __shared__ int bad[2][GBM];
     if (tid < GBM) bad[0][tid] = bad[1][tid] = 0;
     __syncthreads();
-    const int mine = (TA::real ? (BF & OP_H) != 0 : !(AF & OP_H)) ? tid / GBK : tid % GBM;
+    const int mine = (TA::real ? (BF & OP_T) != 0 : !(AF & OP_T)) ? tid / GBK : tid % GBM;
     if (top_im >= 0x7ff00000) bad[0][mine] = 1;
     if (top_re >= 0x7ff00000) bad[1][mine] = 1;
     __syncthreads();
@@ -269,7 +272,9 @@ __global__ __launch_bounds__(GNT, 6) void k_zgemm_mfma(const void* __restrict__ 
       const int ml = wm + 16 * t + 4 * e + kq, nl = wn + i;
       const int m = m0 + ml, n = n0 + nl;
       if (m < M && n < N) {
-        const double re = apply_epi(ep, M, N, m, n, make_double2(cr[t][e], ci[t][e]));
+        double2 v = make_double2(cr[t][e], ci[t][e]);
+        if (MODE == EPI_STORE && bt.scale != 1.0) v = cscale(v, bt.scale);
+        const double re = apply_epi(ep, M, N, m, n, v);
         if constexpr (RE)
           if (argmax) stage[ml * 65 + nl] = re;
       }
@@ -298,25 +303,45 @@ __global__ __launch_bounds__(GNT, 6) void k_zgemm_mfma(const void* __restrict__ 
 }
 
 template <int MODE, int AF, int BF>
-static void launch(hipStream_t st, const MfmaPlan& p, const void* A, long lda, const void* B, long ldb, int M, int N,
-                   int K, const Epi& ep, const Argmax& am, double2* ws, uint32_t* cnt) {
-  MITOK_LAUNCH((k_zgemm_mfma<MODE, AF, BF>), dim3((unsigned)p.blocks()), dim3(GNT), 0, st, A, lda, B, ldb, M, N, K,
-               p.whole, p.P, p.kchunk, ep, am, ws, cnt);
+static int launch(hipStream_t st, const MfmaPlan& p, const GemmOpnd& A, const GemmOpnd& B, int M, int N, int K,
+                  const Epi& ep, const Argmax& am, double2* ws, uint32_t* cnt, const MfmaBatch& bt) {
+  MITOK_LAUNCH((k_zgemm_mfma<MODE, AF, BF>), dim3((unsigned)p.blocks(), (unsigned)bt.n), dim3(GNT), 0, st, A.p, A.ld,
+               B.p, B.ld, M, N, K, p.whole, p.P, p.kchunk, ep, am, ws, cnt, bt);
+  return OK;
 }
 
-int launch_zgemm_mfma(hipStream_t st, const MfmaPlan& p, const double2* A, long lda, bool a_real, const double2* W,
-                      long ldw, int M, int N, int K, const Epi& ep, const Argmax& am, double2* ws, uint32_t* cnt) {
-#define MITOK_CASE(MODE)                                                                    \
-  case MODE:                                                                                \
-    if (a_real) launch<MODE, OP_RE, 0>(st, p, A, lda, W, ldw, M, N, K, ep, am, ws, cnt);    \
-    else launch<MODE, 0, 0>(st, p, A, lda, W, ldw, M, N, K, ep, am, ws, cnt);               \
-    return OK;
-  switch (ep.mode) {
-    MITOK_CASE(EPI_STORE)
-    MITOK_CASE(EPI_GELU)
-    MITOK_CASE(EPI_RE)
-    MITOK_CASE(EPI_QKV)
-    default: return ERR_ARG;  // split partials are for the skinny products
+int launch_zgemm_mfma(hipStream_t st, const MfmaPlan& p, const GemmOpnd& A, const GemmOpnd& B, int M, int N, int K,
+                      const Epi& ep, const Argmax& am, double2* ws, uint32_t* cnt, const MfmaBatch& bt) {
+  if (bt.n < 1 || bt.n > 65535 || (bt.n > 1 && p.P > 1)) return ERR_ARG;  // a batch has no split workspace
+  const auto key = [](int mode, int a, int b) { return mode << 8 | a << 4 | b; };
+#define MITOK_CASE(MODE, AF, BF) \
+  case MODE << 8 | (AF) << 4 | (BF): return launch<MODE, AF, BF>(st, p, A, B, M, N, K, ep, am, ws, cnt, bt);
+  switch (key(ep.mode, A.flags, B.flags)) {
+    // the forward pass: rows times weights
+    MITOK_CASE(EPI_STORE, 0, 0)
+    MITOK_CASE(EPI_STORE, OP_RE, 0)
+    MITOK_CASE(EPI_GELU, 0, 0)
+    MITOK_CASE(EPI_GELU, OP_RE, 0)
+    MITOK_CASE(EPI_RE, 0, 0)
+    MITOK_CASE(EPI_RE, OP_RE, 0)
+    MITOK_CASE(EPI_QKV, 0, 0)
+    MITOK_CASE(EPI_QKV, OP_RE, 0)
+    // weight gradients conj(X)^T G
+    MITOK_CASE(EPI_STORE, OP_H, 0)
+    MITOK_CASE(EPI_STORE, OP_H | OP_RE, 0)
+    MITOK_CASE(EPI_STORE, OP_H, OP_RE)
+    MITOK_CASE(EPI_STORE, OP_H, OP_F64)
+    // input gradients G conj(W)^T
+    MITOK_CASE(EPI_STORE, 0, OP_H)
+    MITOK_CASE(EPI_STORE, OP_RE, OP_H)
+    MITOK_CASE(EPI_STORE, OP_F64, OP_H)
+    // attention: Re(Q K^T), Re(G conj(V)^T), dA conj(K), dA^T conj(Q), A^T G
+    MITOK_CASE(EPI_RE, 0, OP_T)
+    MITOK_CASE(EPI_RE, 0, OP_H)
+    MITOK_CASE(EPI_STORE, OP_F64, OP_CJ)
+    MITOK_CASE(EPI_STORE, OP_F64 | OP_T, OP_CJ)
+    MITOK_CASE(EPI_STORE, OP_F64 | OP_T, 0)
+    default: return ERR_ARG;
   }
 #undef MITOK_CASE
 }

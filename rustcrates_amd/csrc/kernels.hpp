@@ -85,6 +85,7 @@ struct Epi {
   double* hist_re = nullptr;       // RE: also hist_re[hist_cnt[0]][m][n] (logits history, ld N)
   const int* hist_cnt = nullptr;
   const uint32_t* row_mask = nullptr;  // GELU: rows with mask 0 become 0
+  double2* pre = nullptr;              // GELU: also pre[m][n] = v + bias, as backward reads it (ld ldo)
   int check_finite = 0;
   uint32_t* err = nullptr;
   // EPI_QKV: row m = b * S + s
@@ -126,58 +127,6 @@ constexpr int GEMM_PART_MAX_M = 64;
 // The prologue alone: out[m][k] = rowops(x)[m][k]  (materialises a pending row transform)
 void rowops_apply(hipStream_t st, int M, int K, const RowOps& ro, double2* out, long ldo);
 
-// ---- the output head's training step (train.hip) ----
-struct TrainStep {
-  int first = 0;      // the first update: clipped gradient descent (linear_layer.rs:159-174)
-  double lr = 0.0;    // the layer's learning rate
-  double batch = 1;   // sequences in the batch (the descent divides by it)
-  int time_step = 0;  // AdamW's bias-correction step (at least 1)
-};
-// G[r][c] (complex, im 0) = tgt[r] < 0 ? 0 : (P[r][c] - [c == tgt[r]]) / norm[r / S]
-void softmax_grad(hipStream_t st, const double* P, int rows, int V, const int* tgt, const double* norm, int S,
-                  double2* G);
-// cross_entropy_loss_batch of P [B][S][V] for targets [B][T] (tlen[b] each):
-// part [B] the sequences' losses, out [2] the batch loss (re, im); T <= CE_MAX_T
-constexpr int CE_MAX_T = 8192;
-void cross_entropy(hipStream_t st, const double* P, int B, int S, int V, const uint32_t* tgt, const uint32_t* tlen,
-                   int T, double* part, double* out);
-// G = mask[r] ? dH * conj(GELU'(Z)) : 0 (layer.rs:181-192, derivative.rs:48-84); mask may be null (all rows)
-void gelu_backward(hipStream_t st, const double2* dH, const double2* Z, const uint32_t* mask, long rows, int F,
-                   double2* G);
-// out [C][R] = conj(in)^T for in [R][C]
-void conj_transpose(hipStream_t st, const double2* in, long R, long C, double2* out);
-// db [V] = sum_b sum_s G[b][s][:] (per-sequence sums in row order, then in sequence order); ws [B][V]
-void bias_grad(hipStream_t st, const double2* G, int B, int S, int V, double2* ws, double2* db);
-// W [n], b [V] updated in place from dW, db (moments mW, vW, mb, vb)
-void linear_update(hipStream_t st, double2* W, const double2* dW, double2* mW, double2* vW, long n, double2* b,
-                   const double2* db, double2* mb, double2* vb, int V, const TrainStep& ts);
-// the Norm's backward per row of x (or Re(x + resid) + 0i); dx real rows, pg = dout * x_hat
-void norm_backward(hipStream_t st, const double2* x, const double2* resid, long rows, int n, double eps,
-                   const double2* gamma, const double2* beta, const double2* dout, double2* dx, double2* pg);
-// out[j] = mult * (sum over sequences b of the row sum of X[b][:][j]), as bias_grad; ws [B][n]
-void colsum(hipStream_t st, const double2* X, int B, int S, int n, double mult, double2* ws, double2* out);
-// attention weights A and dl_da [B][H][S][S] of a stateless pass from the packed [q | k | v] rows and the
-// gradient G [B*S][d] of the heads' output
-void attn_probs_grad(hipStream_t st, const double2* qkv, const double* bias_re, int mc, const uint32_t* mask,
-                     const double2* G, int B, int S, int H, int dh, double c, double* A, double* dA);
-// the gradient of the packed [q | k | v] rows: dQ = c dA conj(K), dK = c dA^T conj(Q), dV = A^T G
-void attn_dqkv(hipStream_t st, const double2* qkv, const double* A, const double* dA, const double2* G, int B, int S,
-               int H, int dh, double c, double2* dqkv);
-// Re(bias_pos)[h][:S][:S] updated from dA summed over the batch (zero moments each call)
-void attn_bias_update(hipStream_t st, double* bias_re, int mc, const double* dA, int B, int H, int S,
-                      const TrainStep& ts);
-// w [n] updated in place (weight: AdamW's EPSILON floor on v_hat's norm)
-void param_update(hipStream_t st, double2* w, const double2* g, double2* m, double2* v, long n, bool weight,
-                  const TrainStep& ts);
-// RoPE's backward on rows [rows][d] of sequences of S rows (cs: the forward's table)
-void rope_backward(hipStream_t st, const double2* G, long rows, int S, int d, const double2* cs, double2* out);
-// the wavelet layer's backward: out [B][Sin][d] from G [B][S2][d] through a tap table [Sin][4]
-void dwt_backward(hipStream_t st, const double2* G, int B, int S2, int Sin, int d, const int* src, const double* w,
-                  double2* out);
-// the embedding rows of n_ids distinct ids, each with occurrences occ[start[u] .. start[u+1]) (rows of G)
-void embedding_update(hipStream_t st, double2* table, int d, const uint32_t* ids, int n_ids, const int* start,
-                      const int* occ, const double2* G, double lr, double bs, uint32_t* err);
-
 // ---- attention ----
 struct Attn {
   const double2* q = nullptr;  // [B*S][ldq]; head h at column h*dh
@@ -209,18 +158,6 @@ bool attention_prefill(hipStream_t st, const Attn& a);
 // npart partials (row b at q + b * ldq, partial stride part_stride); with
 // `append` the partials are [q | k | v] of the new token, whose k and v the
 // kernel appends to the cache (kc_w, vc_w).
-// MFMA-tiled GEMM (gemm_mfma.hip) for M > 64: block tile GBM x GBN, K step
-// GBK; the first `whole` output tiles are one block each, the `rest` P blocks
-// of kchunk of K.  a_real: A's imaginary parts are zero.  ERR_ARG for EPI_PART.
-constexpr int GBM = 64, GBN = 64, GBK = 8;
-struct MfmaPlan {
-  int whole = 0, rest = 0, P = 1, kchunk = 0;
-  long blocks() const { return whole + (long)rest * P; }
-  size_t ws_bytes() const { return P > 1 ? (size_t)rest * P * GBM * GBN * sizeof(double2) : 0; }
-};
-int launch_zgemm_mfma(hipStream_t st, const MfmaPlan& p, const double2* A, long lda, bool a_real, const double2* W,
-                      long ldw, int M, int N, int K, const Epi& ep, const Argmax& am, double2* ws, uint32_t* cnt);
-
 AttnSplit attention_split_plan(const Attn& a);
 size_t attention_split_ws_bytes(int B, int H, int dh, int T_max);
 int attention_decode_split(hipStream_t st, const Attn& a, const double2* q, long ldq, int npart, long part_stride,
@@ -341,9 +278,6 @@ void layernorm(hipStream_t st, const double2* x, const double2* before, double2*
 void gather_rows(hipStream_t st, const double2* src, int S, int d, const uint32_t* lens, int B, double2* dst);
 // argmax per row with last-index ties (greedy_decoding on host-provided logits)
 void argmax_rows(hipStream_t st, const double* logits, int rows, int V, uint32_t* ids, uint32_t* err);
-void softmax_rows(hipStream_t st, const double2* logits, int rows, int S, int V, const uint32_t* row_mask, int mode,
-                  double* out);
-
 // ---- initialisation ----
 void fill_seeded(hipStream_t st, double2* dst, int rows, int cols, long ld, uint64_t key, double lim);
 void fill_seeded_re(hipStream_t st, double* dst, int rows, int cols, long ld, uint64_t key, double lim);

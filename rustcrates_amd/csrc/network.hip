@@ -21,7 +21,7 @@
 #include <vector>
 
 #include "../../include/mitok.h"
-#include "kernels.hpp"
+#include "train.hpp"
 
 namespace mitok {
 
@@ -327,7 +327,7 @@ struct mitok_network {
   std::vector<uint32_t> kv_len_h;
   mitok::DevBuf kv_len_d, err_d;
   // workspaces
-  mitok::DevBuf act0, act1, qbuf, concat, hbuf, gath, mat0, mat1, logits_c, logits_re, probs, kv_scratch;
+  mitok::DevBuf act0, act1, qbuf, concat, hbuf, gath, mat0, mat1, logits_re, probs, kv_scratch;
   mitok::DevBuf ids_d, mask_d, lens_d, pos_d, kv_row_d, ones_d, dec_ids_d, hist_d, cnt_d, logit_hist_d;
   // split-completion counters (zeroed once, self-resetting), split partials, argmax partials
   mitok::DevBuf sync_cnt, sync_ws, am_v, am_i;
@@ -593,7 +593,6 @@ static int prepare(Net* n, const Spec& sp) {
       const int Mv = (vocab && sp.last_row) ? sp.B : M;
       ws = std::max(ws, gemm_ws_bytes(Mv, L->d_out, L->d_in));
       if (vocab && !sp.forward_only) {
-        TRY(reserve(n, n->logits_c, (size_t)Mv * L->d_out * c16));
         TRY(reserve(n, n->probs, (size_t)Mv * L->d_out * sizeof(double)));
       }
       if (vocab && sp.forward_only) {
@@ -866,8 +865,10 @@ static int enqueue_forward(Net* n, const Spec& sp) {
           TRY(launch_rc(gemm(st, M, Ln->d_out, Ln->d_in, rows_of(x, Ln->d_in, real), Ln->w.as<double2>(), Ln->d_out, e,
                              sp.am, sy), "vocab"));
         } else {
-          e.mode = EPI_STORE;
-          e.out = n->logits_c.as<double2>();
+          // SoftmaxLayer reads the logits' real parts only
+          // (softmax_output_layer.rs:40-64), so only they are formed
+          e.mode = EPI_RE;
+          e.out_re = sp.out_prob;
           TRY(launch_rc(gemm(st, M, Ln->d_out, Ln->d_in, rows_of(x, Ln->d_in, real), Ln->w.as<double2>(), Ln->d_out, e,
                              nullptr, sy), "vocab"));
           if (sp.mode == MODE_STATELESS && !sp.last_row) {  // the layer keeps its input for backward
@@ -879,8 +880,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
             n->head_S = (uint32_t)S;
           }
           auto* SM = (SoftmaxLayer*)n->layers.back().get();
-          softmax_rows(st, n->logits_c.as<double2>(), M, S, Ln->d_out, mask, SM->mode == MITOK_TRAINING ? 0 : 1,
-                       sp.out_prob);
+          softmax_rows(st, sp.out_prob, M, S, Ln->d_out, mask, SM->mode == MITOK_TRAINING ? 0 : 1);
         }
         break;
       }

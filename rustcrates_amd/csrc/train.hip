@@ -13,7 +13,7 @@
 //   update: the first update descends by lr * clip(g) / B where finite; later
 //        ones run AdamW on the unclipped grouped gradient (AdamW clips each
 //        element to norm 1 itself), moments kept per parameter.
-#include "kernels.hpp"
+#include "train.hpp"
 
 namespace mitok {
 
