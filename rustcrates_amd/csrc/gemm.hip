@@ -1222,8 +1222,8 @@ int gemm_tiled(hipStream_t st, int M, int N, int K, const GemmOpnd& A, const Gem
   if (M <= 0 || N <= 0 || bt.n <= 0) return OK;
   if (K <= 0) return ERR_ARG;
   MfmaPlan p = plan_mfma(M, N, K);
-  if (bt.n > 1) p = MfmaPlan{cdiv_i(M, GBM) * cdiv_i(N, GBN)};  // the batch fills the chip
-  if (p.ws_bytes() > sy.ws_bytes) return ERR_STATE;
+  // a batch fills the chip by itself (and has no split workspace)
+  if (bt.n > 1 || p.ws_bytes() > sy.ws_bytes) p = MfmaPlan{cdiv_i(M, GBM) * cdiv_i(N, GBN)};
   return launch_zgemm_mfma(st, p, A, B, M, N, K, ep, Argmax(), (double2*)sy.ws, sy.counters, bt);
 }
 

@@ -392,7 +392,8 @@ struct mitok_network {
   // what a stateless pass keeps for backward: each layer's input rows, and
   // the heads' output of each SelfAttention layer (before its residual + Norm)
   std::vector<std::unique_ptr<mitok::DevBuf>> tr_in, tr_cat;
-  mitok::DevBuf tr_g, tr_xh, tr_wh, tr_dw, tr_db, tr_ga, tr_gb, tr_tgt, tr_norm;
+  std::vector<char> tr_real;  // whether a layer's input rows had zero imaginary parts
+  mitok::DevBuf tr_g, tr_xh, tr_dw, tr_db, tr_ga, tr_gb, tr_tgt, tr_norm;
   mitok::DevBuf tr_z, tr_h, tr_g1, tr_dh, tr_qkv, tr_dqkv, tr_A, tr_dA, tr_pg, tr_eid, tr_est, tr_eocc, tr_bsum;
   mitok::DevBuf ce_buf;  // mitok_cross_entropy_loss: targets, lengths, per-sequence losses, the result
 };
@@ -572,6 +573,7 @@ static int prepare(Net* n, const Spec& sp) {
   if (sp.mode == MODE_STATELESS) {  // the layer inputs backward reads
     while (n->tr_in.size() < n->layers.size()) n->tr_in.push_back(std::make_unique<DevBuf>());
     while (n->tr_cat.size() < n->layers.size()) n->tr_cat.push_back(std::make_unique<DevBuf>());
+    n->tr_real.assign(n->layers.size(), 0);
     for (uint32_t li = sp.first; li < sp.last; ++li) {
       const Layer* L = n->layers[li].get();
       if (L->kind != K_EMBEDDING && L->kind != K_SOFTMAX) TRY(reserve(n, *n->tr_in[li], rows * L->d_in * c16));
@@ -692,6 +694,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
     Layer* L = n->layers[li].get();
     if (sp.mode == MODE_STATELESS && L->kind != K_EMBEDDING && L->kind != K_SOFTMAX)  // kept for backward
       HIP_TRY(hipMemcpyAsync(n->tr_in[li]->p, cur, (size_t)rows * L->d_in * sizeof(double2), hipMemcpyDeviceToDevice, st));
+    if (sp.mode == MODE_STATELESS) n->tr_real[li] = real;
     switch (L->kind) {
       case K_EMBEDDING: {
         auto* E = (EmbeddingLayer*)L;
@@ -2837,7 +2840,10 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
   std::vector<std::vector<double>> keep_d;
   // what the walk needs, checked and sized before the first launch
   size_t dmax = (size_t)d, fmax = 0, d3max = 0, att = 0, wmax = (size_t)d * V, bmax = (size_t)V;
-  size_t ws = std::max(gemm_ws_bytes(d, V, (int)rows), gemm_ws_bytes((int)rows, d, V));
+  size_t ws = 0;
+  const auto linear_ws = [&](long r, int din, int dout) {  // linear_bwd's two products
+    ws = std::max({ws, gemm_tiled_ws_bytes(din, dout, (int)r), gemm_tiled_ws_bytes((int)r, din, dout)});
+  };
   for (uint32_t li = stop; li < li_top; ++li) {
     const Layer* L = n->layers[li].get();
     const int di = (int)L->d_in, dn = (int)L->d_out;
@@ -2853,28 +2859,29 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
       case K_LINEAR:
         wmax = std::max(wmax, (size_t)di * dn);
         bmax = std::max(bmax, (size_t)dn);
-        ws = std::max({ws, gemm_ws_bytes(di, dn, (int)rows), gemm_ws_bytes((int)rows, di, dn)});
+        linear_ws(rows, di, dn);
         break;
       case K_FEED_FORWARD: {
         const int F = (int)((const FeedForwardLayer*)L)->hidden;
         fmax = std::max(fmax, (size_t)F);
         wmax = std::max(wmax, (size_t)di * F);
         bmax = std::max(bmax, (size_t)F);
-        ws = std::max({ws, gemm_ws_bytes((int)rows, F, di), gemm_ws_bytes(F, dn, (int)rows),
-                       gemm_ws_bytes((int)rows, F, dn), gemm_ws_bytes(di, F, (int)rows), gemm_ws_bytes((int)rows, di, F)});
+        ws = std::max(ws, gemm_ws_bytes((int)rows, F, di));
+        linear_ws(rows, F, dn);
+        linear_ws(rows, di, F);
         break;
       }
       case K_SELF_ATTENTION: {
         const auto* A = (const SelfAttentionLayer*)L;
         if ((uint32_t)S > A->max_ctx) return fail(ERR_ARG, "layer %u: %d rows exceed max context %u", li, S, A->max_ctx);
-        // k_attn_probs_grad holds a query row's weights and Re(dl_ds) in LDS (2 S doubles beside 6 KB)
+        // k_attn_probs_grad holds a query row's weights and Re(dl_ds) in registers
         if (S > 3072) return fail(ERR_ARG, "layer %u: attention backward of %d rows (at most 3072)", li, S);
         if (A->dh > 256) return fail(ERR_ARG, "layer %u: attention backward of %u-wide heads (at most 256)", li, A->dh);
         d3max = std::max(d3max, (size_t)3 * di);
         att = std::max(att, (size_t)A->heads * S * S);
         wmax = std::max(wmax, (size_t)3 * di * di);
-        ws = std::max({ws, gemm_ws_bytes((int)rows, 3 * di, di), gemm_ws_bytes(di, 3 * di, (int)rows),
-                       gemm_ws_bytes((int)rows, di, 3 * di)});
+        ws = std::max(ws, gemm_ws_bytes((int)rows, 3 * di, di));
+        linear_ws(rows, di, 3 * di);
         break;
       }
       default: break;
@@ -2904,6 +2911,29 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
       tgt[(size_t)b * S + s] = (int)tc;
     }
   }
+  // The rows with a target, packed in order, and one zero row for the others
+  // (every sequence has some: its last row predicts nothing): a target-less
+  // row's gradient is zero, so the head's products skip it.
+  // ints: [rows] target, [rows] packed row, [packed] output row (-1: zero), [B + 1] first packed row of a sequence
+  std::vector<int> head(2 * (size_t)rows);
+  int packed = 0;
+  {
+    std::vector<int> list, starts(1, 0);
+    for (long r = 0; r < rows; ++r) {
+      head[r] = tgt[r];
+      head[rows + r] = tgt[r] >= 0 ? (int)list.size() : -1;
+      if (tgt[r] >= 0) list.push_back((int)r);
+      if ((r + 1) % S == 0) starts.push_back((int)list.size());
+    }
+    for (long r = 0; r < rows; ++r)
+      if (head[rows + r] < 0) head[rows + r] = (int)list.size();
+    list.push_back(-1);
+    packed = (int)list.size();
+    head.insert(head.end(), list.begin(), list.end());
+    head.insert(head.end(), starts.begin(), starts.end());
+  }
+  linear_ws(packed, d, V);
+  if (packed > 1) linear_ws(packed - 1, d, V);
   // EmbeddingLayer::update_parameters' order: sequence by sequence, target by
   // target; grouped per id (a repeated id applies its rows in that order)
   const bool embed_upd = update_params && stop == 0 && n->layers[0]->kind == K_EMBEDDING;
@@ -2966,18 +2996,17 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
     TRY(upload(n, W.gw, keep_d.back().data(), keep_d.back().size() * sizeof(double)));
   }
   // every workspace is sized before the first launch (a reserve that grows frees the old buffer)
-  TRY(upload(n, n->tr_tgt, tgt.data(), tgt.size() * sizeof(int)));
+  TRY(upload(n, n->tr_tgt, head.data(), head.size() * sizeof(int)));
   TRY(upload(n, n->tr_norm, norm.data(), norm.size() * sizeof(double)));
   if (embed_upd && !eids.empty()) {
     TRY(upload(n, n->tr_eid, eids.data(), eids.size() * sizeof(uint32_t)));
     TRY(upload(n, n->tr_est, estart.data(), estart.size() * sizeof(int)));
     TRY(upload(n, n->tr_eocc, eocc.data(), eocc.size() * sizeof(int)));
   }
-  TRY(reserve(n, n->tr_g, (size_t)rows * V * c16));
+  TRY(reserve(n, n->tr_g, (size_t)packed * V * sizeof(double)));
   TRY(reserve(n, n->tr_ga, (size_t)rows_max * dmax * c16));
   TRY(reserve(n, n->tr_gb, (size_t)rows_max * dmax * c16));
-  TRY(reserve(n, n->tr_xh, (size_t)rows_max * std::max(dmax, fmax) * c16));
-  TRY(reserve(n, n->tr_wh, wmax * c16));
+  TRY(reserve(n, n->tr_xh, (size_t)2 * packed * d * c16));  // packed head input, packed input gradient
   TRY(reserve(n, n->tr_dw, wmax * c16));
   TRY(reserve(n, n->tr_db, std::max(bmax, dmax) * c16));
   TRY(reserve(n, n->tr_dh, (size_t)rows_max * std::max(fmax, dmax) * c16));
@@ -3018,25 +3047,33 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
   long rows_c = rows;  // the current layer's rows (a wavelet layer changes them below it)
   int S_c = S;
   const uint32_t* mask_c = n->head_mask;
-  double2* xh = n->tr_xh.as<double2>();
-  double2* wh = n->tr_wh.as<double2>();
   double2* dW = n->tr_dw.as<double2>();
   double2* db = n->tr_db.as<double2>();
-  // LinearLayer::backward, complex arm (linear_layer.rs:96-108), grouped over
-  // the sequences: dW = conj(X)^T G, db = column sums, dX = G conj(W)^T
-  auto linear_bwd = [&](const double2* X, const double2* G, const double2* W, int din, int dout, double2* dX) -> int {
-    conj_transpose(st, X, rows_c, din, xh);
+  double2* bsum = n->tr_bsum.as<double2>();
+  // dW = conj(X)^T G and dX = G conj(W)^T (linear_layer.rs:96-108) of `r` rows,
+  // xf / gf: the operand flags of X and G (at most one of them real)
+  auto grads = [&](const double2* X, int xf, const void* G, int gf, const double2* W, long r, int din, int dout,
+                   double2* dX, bool last_zero = false) -> int {
+    if (gf) xf = 0;
     Epi e;
     e.mode = EPI_STORE;
     e.err = err;
     e.out = dW;
     e.ldo = dout;
-    TRY(launch_rc(gemm(st, din, dout, (int)rows_c, rows_of(xh, rows_c), G, dout, e, nullptr, sy), "weight grad"));
-    bias_grad(st, G, (int)B, S_c, dout, n->tr_bsum.as<double2>(), db);
-    conj_transpose(st, W, din, dout, wh);
+    TRY(launch_rc(gemm_tiled(st, din, dout, (int)r, GemmOpnd{X, din, OP_H | xf}, GemmOpnd{G, dout, gf}, e, sy),
+                  "weight grad"));
     e.out = dX;
     e.ldo = din;
-    TRY(launch_rc(gemm(st, (int)rows_c, din, dout, rows_of(G, dout), wh, din, e, nullptr, sy), "input grad"));
+    MfmaBatch bt;
+    if (last_zero && r > 1) bt.zero_row = dX + --r * din;  // without a tile for the last row, which is zero
+    TRY(launch_rc(gemm_tiled(st, (int)r, din, dout, GemmOpnd{G, dout, gf}, GemmOpnd{W, dout, OP_H}, e, sy, bt), "input grad"));
+    return OK;
+  };
+  // LinearLayer::backward, complex arm, grouped over the sequences; db = column sums
+  auto linear_bwd = [&](const double2* X, bool xreal, const double2* G, bool greal, const double2* W, int din, int dout,
+                        double2* dX) -> int {
+    TRY(grads(X, xreal ? OP_RE : 0, G, greal ? OP_RE : 0, W, rows_c, din, dout, dX));
+    colsum(st, G, (int)B, S_c, dout, 1.0, bsum, db);
     return OK;
   };
   // update_parameters of a weight and its bias from dW, db (linear_layer.rs:130-175)
@@ -3052,16 +3089,27 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
                   mb.as<double2>(), vb.as<double2>(), nb, ts);
     updates++;
   };
-  double2* G = n->tr_g.as<double2>();
-  softmax_grad(st, n->probs.as<double>(), (int)rows, V, n->tr_tgt.as<int>(), n->tr_norm.as<double>(), S, G);
   double2* gcur = n->tr_ga.as<double2>();  // the gradient of the current layer's output, then its input
   double2* gnext = n->tr_gb.as<double2>();
-  TRY(linear_bwd(n->head_x, G, Ln->w.as<double2>(), d, V, gcur));
+  bool greal = false;  // gcur's imaginary parts are zero: a Norm's backward leaves real gradients (norm_layer.rs:132-209)
+  {
+    const int* tgt_d = n->tr_tgt.as<int>();
+    const int *packed_d = tgt_d + rows, *list_d = packed_d + rows, *starts_d = list_d + packed;
+    double* G = n->tr_g.as<double>();
+    double2 *X = n->tr_xh.as<double2>(), *dX = X + (size_t)packed * d;
+    softmax_grad(st, n->probs.as<double>(), packed, V, list_d, tgt_d, n->tr_norm.as<double>(), S, G);
+    pack_rows(st, n->head_x, rows, d, packed_d, packed - 1, X);
+    fill_const(st, dX + (size_t)(packed - 1) * d, d, make_double2(0.0, 0.0));
+    TRY(grads(X, 0, G, OP_F64, Ln->w.as<double2>(), packed, d, V, dX, true));
+    colsum_packed(st, G, starts_d, (int)B, V, bsum, db);
+    unpack_rows(st, dX, rows, d, packed_d, gcur);
+  }
   if (update_params)
     linear_upd(Ln->w, Ln->b, (long)d * V, V, Ln->mw, Ln->vw, Ln->mb, Ln->vb, Ln->updates, (int)time_step, rate(Ln));
   for (int li = (int)li_top - 1; li >= (int)stop; --li) {
     Layer* L = n->layers[li].get();
     const double2* X = n->tr_in[li]->as<double2>();
+    const bool xreal = n->tr_real[li] != 0;
     const uint32_t* mask = mask_c;
     if (!stage_at[li]) {  // every other layer keeps its rows
       S_c = S_in_at[li];
@@ -3081,10 +3129,11 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
       }
       case K_LINEAR: {
         auto* H = (LinearLayer*)L;
-        TRY(linear_bwd(X, gcur, H->w.as<double2>(), H->d_in, H->d_out, gnext));
+        TRY(linear_bwd(X, xreal, gcur, greal, H->w.as<double2>(), H->d_in, H->d_out, gnext));
         if (update_params) linear_upd(H->w, H->b, (long)H->d_in * H->d_out, H->d_out, H->mw, H->vw, H->mb, H->vb, H->updates,
                                       (int)time_step, rate(H));
         std::swap(gcur, gnext);
+        greal = false;
         break;
       }
       case K_FEED_FORWARD: {
@@ -3099,21 +3148,22 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
         e.mode = EPI_GELU;  // the Dense output the forward pass gave its Linear: GELU, padded rows 0
         e.row_mask = mask;
         e.out = n->tr_h.as<double2>();
-        TRY(launch_rc(gemm(st, (int)rows, Fh, di, rows_of(X, di), F->w1.as<double2>(), Fh, e, nullptr, sy), "ffn1 output"));
+        TRY(launch_rc(gemm(st, (int)rows, Fh, di, rows_of(X, di, xreal), F->w1.as<double2>(), Fh, e, nullptr, sy), "ffn1 output"));
         e.mode = EPI_STORE;  // its pre-activation Z = X W1 + b1 (layer.rs:135-144)
         e.row_mask = nullptr;
         e.out = n->tr_z.as<double2>();
-        TRY(launch_rc(gemm(st, (int)rows, Fh, di, rows_of(X, di), F->w1.as<double2>(), Fh, e, nullptr, sy),
+        TRY(launch_rc(gemm(st, (int)rows, Fh, di, rows_of(X, di, xreal), F->w1.as<double2>(), Fh, e, nullptr, sy),
                       "ffn1 pre-activation"));
-        TRY(linear_bwd(n->tr_h.as<double2>(), gcur, F->w2.as<double2>(), Fh, dn, n->tr_dh.as<double2>()));
+        TRY(linear_bwd(n->tr_h.as<double2>(), false, gcur, greal, F->w2.as<double2>(), Fh, dn, n->tr_dh.as<double2>()));
         // FeedForwardLayer::update_parameters (:219-250): the Linear at the FFN's time step (:86)
         if (update_params) linear_upd(F->w2, F->b2, (long)Fh * dn, dn, F->mw2, F->vw2, F->mb2, F->vb2, F->updates2,
                                       (int)time_step, rate(F));
         gelu_backward(st, n->tr_dh.as<double2>(), n->tr_z.as<double2>(), mask, rows, Fh, n->tr_g1.as<double2>());
-        TRY(linear_bwd(X, n->tr_g1.as<double2>(), F->w1.as<double2>(), di, Fh, gnext));
+        TRY(linear_bwd(X, xreal, n->tr_g1.as<double2>(), false, F->w1.as<double2>(), di, Fh, gnext));
         // the Dense at step 1: Layer::time_step stays 0 after construction (layer.rs:111,285)
         if (update_params) linear_upd(F->w1, F->b1, (long)di * Fh, Fh, F->mw1, F->vw1, F->mb1, F->vb1, F->updates1, 0, rate(F));
         std::swap(gcur, gnext);
+        greal = false;
         break;
       }
       case K_SELF_ATTENTION: {
@@ -3126,29 +3176,64 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
         double2* gn = n->tr_dh.as<double2>();
         norm_backward(st, n->tr_cat[li]->as<double2>(), X, rows, da, A->eps, A->gamma.as<double2>(), A->beta.as<double2>(),
                       gcur, gn, n->tr_pg.as<double2>());
+        // q rows [rows][da], then k and v as the forward pass holds them, [B][H][S][dh]
+        double2 *q = n->tr_qkv.as<double2>(), *k = q + (size_t)rows * da, *v = k + (size_t)rows * da;
         Epi e;
-        e.mode = EPI_STORE;
+        e.mode = EPI_QKV;
         e.err = err;
-        e.out = n->tr_qkv.as<double2>();
-        e.ldo = 3 * da;
-        TRY(launch_rc(gemm(st, (int)rows, 3 * da, da, rows_of(X, da), A->wqkv.as<double2>(), 3 * da, e, nullptr, sy),
-                      "qkv"));
-        attn_probs_grad(st, n->tr_qkv.as<double2>(), A->bias_re.as<double>(), mc, mask, gn, (int)B, S, H, dh, c,
-                        n->tr_A.as<double>(), n->tr_dA.as<double>());
-        attn_dqkv(st, n->tr_qkv.as<double2>(), n->tr_A.as<double>(), n->tr_dA.as<double>(), gn, (int)B, S, H, dh, c,
-                  n->tr_dqkv.as<double2>());
-        // the heads' weight gradients grouped over the batch: conj(X)^T [dq | dk | dv]
-        conj_transpose(st, X, rows, da, xh);
-        e.out = dW;
-        e.ldo = 3 * da;
-        TRY(launch_rc(gemm(st, da, 3 * da, (int)rows, rows_of(xh, rows), n->tr_dqkv.as<double2>(), 3 * da, e, nullptr, sy),
-                      "qkv weight grad"));
-        // the heads' input gradients summed: [dq | dk | dv] conj([Wq | Wk | Wv])^T
-        conj_transpose(st, A->wqkv.as<double2>(), da, 3 * da, wh);
-        e.out = gnext;
+        e.out = q;
         e.ldo = da;
-        TRY(launch_rc(gemm(st, (int)rows, da, 3 * da, rows_of(n->tr_dqkv.as<double2>(), 3 * da), wh, da, e, nullptr, sy),
-                      "qkv input grad"));
+        e.d = da;
+        e.dh = dh;
+        e.heads = H;
+        e.S = S;
+        e.kc = k;
+        e.vc = v;
+        e.ctx = S;
+        TRY(launch_rc(gemm(st, (int)rows, 3 * da, da, rows_of(X, da, xreal), A->wqkv.as<double2>(), 3 * da, e, nullptr, sy),
+                      "qkv"));
+        // the heads' products, one batch entry per (sequence, head): Re(q.k),
+        // Re(dl_ds), then dQ = c dA conj(K), dK = c dA^T conj(Q), dV = A^T G
+        // (masked_attention_head.rs:276-316) as the gradient of the packed
+        // [q | k | v] rows
+        double *At = n->tr_A.as<double>(), *dAt = n->tr_dA.as<double>();
+        double2* dqkv = n->tr_dqkv.as<double2>();
+        const long SS = (long)S * S, rs = (long)S * da, ks = (long)S * dh;  // steps of a head's S x S, a sequence's rows, a head's keys
+        const auto heads = [&](int M, int N, int K, GemmOpnd a, long a0, long a1, GemmOpnd b, long b0, long b1,
+                               double2* out, double* out_re, long ldo, long c0, long c1, double scale) -> int {
+          Epi h;
+          h.mode = out_re ? EPI_RE : EPI_STORE;
+          h.err = err;
+          h.out = out;
+          h.out_re = out_re;
+          h.ldo = ldo;
+          const size_t sa = a.flags & OP_F64 ? sizeof(double) : c16, total = (size_t)B * H;
+          const size_t most = 65535 / H * H;  // whole sequences of one launch
+          for (size_t z = 0; z < total; z += most) {
+            const long b_ = (long)(z / H);
+            GemmOpnd az = a, bz = b;
+            az.p = (const char*)a.p + b_ * a0 * sa;
+            bz.p = (const double2*)b.p + b_ * b0;
+            Epi hz = h;
+            if (out_re) hz.out_re += b_ * c0;
+            else hz.out += b_ * c0;
+            const MfmaBatch bt{(int)std::min(most, total - z), H, a0, a1, b0, b1, c0, c1, scale};
+            TRY(launch_rc(gemm_tiled(st, M, N, K, az, bz, hz, sy, bt), "attention grad"));
+          }
+          return OK;
+        };
+        TRY(heads(S, S, dh, GemmOpnd{q, da, 0}, rs, dh, GemmOpnd{k, dh, OP_T}, H * ks, ks, nullptr, At, S, H * SS, SS, 1.0));
+        TRY(heads(S, S, dh, GemmOpnd{gn, da, 0}, rs, dh, GemmOpnd{v, dh, OP_H}, H * ks, ks, nullptr, dAt, S, H * SS, SS, 1.0));
+        attn_probs_grad(st, At, dAt, A->bias_re.as<double>(), mc, mask, (int)B, S, H, c);
+        TRY(heads(S, dh, S, GemmOpnd{dAt, S, OP_F64}, H * SS, SS, GemmOpnd{k, dh, OP_CJ}, H * ks, ks, dqkv, nullptr, 3 * da,
+                  3 * rs, dh, c));
+        TRY(heads(S, dh, S, GemmOpnd{dAt, S, OP_F64 | OP_T}, H * SS, SS, GemmOpnd{q, da, OP_CJ}, rs, dh, dqkv + da, nullptr,
+                  3 * da, 3 * rs, dh, c));
+        TRY(heads(S, dh, S, GemmOpnd{At, S, OP_F64 | OP_T}, H * SS, SS, GemmOpnd{gn, da, 0}, rs, dh, dqkv + 2 * da, nullptr,
+                  3 * da, 3 * rs, dh, 1.0));
+        // the heads' weight gradients grouped over the batch and their input
+        // gradients summed: conj(X)^T [dq | dk | dv], [dq | dk | dv] conj([Wq | Wk | Wv])^T
+        TRY(grads(X, xreal ? OP_RE : 0, dqkv, 0, A->wqkv.as<double2>(), rows, da, 3 * da, gnext));
         if (update_params) {  // SelfAttentionLayer::update_parameters (:260-273): the Norm, then the heads
           TrainStep ts;
           ts.lr = rate(A);
@@ -3167,6 +3252,7 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
           A->updates++;
         }
         std::swap(gcur, gnext);
+        greal = false;
         break;
       }
       case K_NORM: {  // NormalNormLayer::backward; the walk does not update a standalone Norm
@@ -3174,6 +3260,7 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
         norm_backward(st, X, nullptr, rows, N->d_in, N->eps, N->gamma.as<double2>(), N->beta.as<double2>(), gcur, gnext,
                       n->tr_pg.as<double2>());
         std::swap(gcur, gnext);
+        greal = true;
         break;
       }
       case K_POSENC: {

@@ -1,14 +1,14 @@
-// train.hip — the output head's training step on gfx950: the kernels around
-// the two products of LinearLayer::backward (linear_layer.rs:77-128) for the
-// vocab Linear behind SoftmaxLayer::backward (softmax_output_layer.rs:67-145),
-// and LinearLayer::update_parameters (linear_layer.rs:130-175) with the
-// reference's AdamW (utils/adam_w.rs:9-103).
+// train.hip — backward's kernels on gfx950 around its tiled products
+// (gemm_mfma.hip): SoftmaxLayer::backward (softmax_output_layer.rs:67-145),
+// LinearLayer::backward's sums (linear_layer.rs:77-128) and update_parameters
+// (:130-175) with the reference's AdamW (utils/adam_w.rs:9-103), and the
+// elementwise and row kernels of the other layers' reverse walk.
 //
-//   G  = softmax gradient, one row per output row; row r of sequence b
-//        holds (p - [c == target]) / (B * non-PAD targets of b) when the
-//        row predicts a target, else 0 (the host maps rows to targets);
-//        stored as complex with im 0, the reference's Complex gradient
-//   dW = conj(X)^T G and dX = G conj(W)^T: gemm() on conjugate transposes
+//   G  = softmax gradient (p - [c == target]) / (B * non-PAD targets of b) of
+//        the rows that predict a target (the host maps rows to targets); the
+//        other rows' is zero.  The head's products run on the target rows
+//        alone, packed, with one zero row standing for all the others
+//   dW = conj(X)^T G and dX = G conj(W)^T, transposes read in place
 //   db = the column sums of G
 //   update: the first update descends by lr * clip(g) / B where finite; later
 //        ones run AdamW on the unclipped grouped gradient (AdamW clips each
@@ -17,65 +17,92 @@
 
 namespace mitok {
 
-// one block per output row: 256 threads stream the row's probabilities
-__global__ __launch_bounds__(256) void k_softmax_grad(const double* __restrict__ P, int V, const int* __restrict__ tgt,
-                                                      const double* __restrict__ norm, int S, double2* __restrict__ G) {
+// Packed row i of the softmax gradient, real: (p - [c == target]) / norm of
+// output row rows[i], or the zero row (rows[i] < 0).  One block per row.
+__global__ __launch_bounds__(256) void k_softmax_grad(const double* __restrict__ P, int V, const int* __restrict__ rows,
+                                                      const int* __restrict__ tgt, const double* __restrict__ norm,
+                                                      int S, double* __restrict__ G) {
+  const long i = blockIdx.x;
+  const int r = rows[i], t = r < 0 ? -1 : tgt[r];
+  const double nz = r < 0 ? 1.0 : norm[r / S];
+  const double* p = P + (long)max(r, 0) * V;
+  double* g = G + i * V;
+  for (int c = threadIdx.x; c < V; c += 256) g[c] = t < 0 ? 0.0 : (c == t ? p[c] - 1.0 : p[c]) / nz;  // softmax_output_layer.rs:128-135
+}
+
+// Packed rows of X beside them: row r goes to packed[r].  The rows without a
+// target share packed row `zero` (zeros before the launch): their gradient is
+// zero, so all they could give a sum is the NaN of 0 * (infinity or NaN).
+__global__ __launch_bounds__(256) void k_pack_rows(const double2* __restrict__ X, int d, const int* __restrict__ packed,
+                                                   int zero, double2* __restrict__ out) {
   const long r = blockIdx.x;
-  const int t = tgt[r];
-  const double nz = norm[r / S];
-  const double* p = P + r * V;
-  double2* g = G + r * V;
-  for (int c = threadIdx.x; c < V; c += 256) {
-    double v = 0.0;
-    if (t >= 0) v = (c == t ? p[c] - 1.0 : p[c]) / nz;  // softmax_output_layer.rs:128-135
-    g[c] = make_double2(v, 0.0);
+  const int i = packed[r];
+  for (int c = threadIdx.x; c < d; c += 256) {
+    const double2 v = X[r * d + c];
+    if (i != zero) {
+      out[(long)i * d + c] = v;
+    } else {
+      if (!isfinite(v.x)) out[(long)i * d + c].x = NAN;
+      if (!isfinite(v.y)) out[(long)i * d + c].y = NAN;
+    }
   }
 }
 
-// out[c][r] = conj(in[r][c]) for in [R][C]: 16x16 tiles through LDS
-__global__ __launch_bounds__(256) void k_conj_transpose(const double2* __restrict__ in, long R, long C,
-                                                        double2* __restrict__ out) {
-  __shared__ double2 t[16][17];
-  const long r0 = (long)blockIdx.y * 16, c0 = (long)blockIdx.x * 16;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  if (r0 + ty < R && c0 + tx < C) {
-    const double2 v = in[(r0 + ty) * C + c0 + tx];
-    t[ty][tx] = make_double2(v.x, -v.y);
+// out[r] = in[packed[r]]: the input gradient of every row from the packed ones
+__global__ __launch_bounds__(256) void k_unpack_rows(const double2* __restrict__ in, int d,
+                                                     const int* __restrict__ packed, double2* __restrict__ out) {
+  const long r = blockIdx.x;
+  const double2* src = in + (long)packed[r] * d;
+  for (int c = threadIdx.x; c < d; c += 256) out[r * d + c] = src[c];
+}
+
+// db[c] = sum over sequences b of (sum over the rows s of b of G[s][c])
+// (linear_layer.rs:101-105, group_gradient_batch_bias).  Bound by the loads in
+// flight: a block takes 64 columns of one sequence, each wave a quarter of its
+// rows, eight loads at a time, the quarters added in row order (8 x 128 rows of
+// 2048: 18 -> 5.5 us against one thread per (sequence, column)).  Then one thread
+// per column adds the sequences in order, times `mult`.  starts: sequence b's
+// rows are [starts[b], starts[b + 1]), or null for S rows each.
+__device__ __forceinline__ double zero_of(double) { return 0.0; }
+__device__ __forceinline__ double2 zero_of(double2) { return make_double2(0.0, 0.0); }
+__device__ __forceinline__ double addt(double a, double b) { return a + b; }
+__device__ __forceinline__ double2 addt(double2 a, double2 b) { return cadd(a, b); }
+template <class T>
+__global__ __launch_bounds__(256) void k_seq_colsum(const T* __restrict__ G, const int* __restrict__ starts, int S,
+                                                    int V, T* __restrict__ part) {
+  __shared__ T quarter[3][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cols = (V + 63) / 64;
+  const int b = blockIdx.x / cols, c = (blockIdx.x - b * cols) * 64 + lane;
+  const int r0 = starts ? starts[b] : b * S, n = (starts ? starts[b + 1] : r0 + S) - r0;
+  const int ra = (int)((long)n * wave / 4), rb = (int)((long)n * (wave + 1) / 4);
+  T s = zero_of(T());
+  if (c < V) {
+    const T* g = G + (long)(r0 + ra) * V + c;
+    int r = ra;
+    for (; r + 8 <= rb; r += 8) {
+      T u[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) u[q] = g[(long)q * V];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) s = addt(s, u[q]);
+      g += 8l * V;
+    }
+    for (; r < rb; ++r, g += V) s = addt(s, g[0]);
   }
+  if (wave) quarter[wave - 1][lane] = s;
   __syncthreads();
-  if (c0 + ty < C && r0 + tx < R) out[(c0 + ty) * R + r0 + tx] = t[tx][ty];
+  if (wave == 0 && c < V) part[(long)b * V + c] = addt(addt(addt(s, quarter[0][lane]), quarter[1][lane]), quarter[2][lane]);
 }
-
-// db[c] = sum over sequences b of (sum over rows s of G[b][s][c]): each
-// sequence's column sum in row order, then the sequences in order
-// (linear_layer.rs:101-105, group_gradient_batch_bias).  Two launches: one
-// thread per (sequence, column) sums its rows (eight loads in flight), then
-// one per column adds the sequences' sums, times `mult`.
-__global__ __launch_bounds__(256) void k_seq_colsum(const double2* __restrict__ G, int B, int S, int V,
-                                                    double2* __restrict__ part) {
-  const long t = (long)blockIdx.x * 256 + threadIdx.x;
-  if (t >= (long)B * V) return;
-  const int c = (int)(t % V), b = (int)(t / V);
-  const double2* g = G + (long)b * S * V + c;
-  double2 s = make_double2(0.0, 0.0);
-  int r = 0;
-  for (; r + 8 <= S; r += 8) {
-    double2 u[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) u[q] = g[(long)(r + q) * V];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) s = cadd(s, u[q]);
-  }
-  for (; r < S; ++r) s = cadd(s, g[(long)r * V]);
-  part[t] = s;
-}
-__global__ __launch_bounds__(256) void k_seq_sum(const double2* __restrict__ part, int B, int V, double mult,
+__device__ __forceinline__ double2 as_complex(double v) { return make_double2(v, 0.0); }
+__device__ __forceinline__ double2 as_complex(double2 v) { return v; }
+template <class T>
+__global__ __launch_bounds__(256) void k_seq_sum(const T* __restrict__ part, int B, int V, double mult,
                                                  double2* __restrict__ out) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= V) return;
-  double2 acc = make_double2(0.0, 0.0);
-  for (int b = 0; b < B; ++b) acc = cadd(acc, part[(long)b * V + c]);
-  out[c] = mult == 1.0 ? acc : cscale(acc, mult);
+  T acc = zero_of(T());
+  for (int b = 0; b < B; ++b) acc = addt(acc, part[(long)b * V + c]);
+  out[c] = mult == 1.0 ? as_complex(acc) : cscale(as_complex(acc), mult);
 }
 
 // f64::powi as compiler-rt's __powidf2 (square and multiply over the bits)
@@ -177,9 +204,18 @@ void gelu_backward(hipStream_t st, const double2* dH, const double2* Z, const ui
   if (n > 0) MITOK_LAUNCH(k_gelu_backward, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, dH, Z, mask, rows, F, G);
 }
 
-void softmax_grad(hipStream_t st, const double* P, int rows, int V, const int* tgt, const double* norm, int S,
-                  double2* G) {
-  if (rows > 0) MITOK_LAUNCH(k_softmax_grad, dim3(rows), dim3(256), 0, st, P, V, tgt, norm, S, G);
+void softmax_grad(hipStream_t st, const double* P, int n, int V, const int* rows, const int* tgt, const double* norm,
+                  int S, double* G) {
+  if (n > 0) MITOK_LAUNCH(k_softmax_grad, dim3(n), dim3(256), 0, st, P, V, rows, tgt, norm, S, G);
+}
+
+void pack_rows(hipStream_t st, const double2* X, long rows, int d, const int* packed, int zero, double2* out) {
+  fill_const(st, out + (long)zero * d, d, make_double2(0.0, 0.0));
+  if (rows > 0) MITOK_LAUNCH(k_pack_rows, dim3((unsigned)rows), dim3(256), 0, st, X, d, packed, zero, out);
+}
+
+void unpack_rows(hipStream_t st, const double2* in, long rows, int d, const int* packed, double2* out) {
+  if (rows > 0) MITOK_LAUNCH(k_unpack_rows, dim3((unsigned)rows), dim3(256), 0, st, in, d, packed, out);
 }
 
 // cross_entropy_loss_batch (transformer_network.rs:662-711) on the softmax
@@ -227,13 +263,18 @@ void cross_entropy(hipStream_t st, const double* P, int B, int S, int V, const u
   MITOK_LAUNCH(k_ce_batch, dim3(1), dim3(64), 0, st, part, B, out);
 }
 
-void conj_transpose(hipStream_t st, const double2* in, long R, long C, double2* out) {
-  const dim3 grid((unsigned)((C + 15) / 16), (unsigned)((R + 15) / 16));
-  if (R > 0 && C > 0) MITOK_LAUNCH(k_conj_transpose, grid, dim3(256), 0, st, in, R, C, out);
+template <class T>
+static void colsum_of(hipStream_t st, const T* X, const int* starts, int B, int S, int n, double mult, void* ws,
+                      double2* out) {
+  if (n <= 0 || B <= 0) return;
+  MITOK_LAUNCH(k_seq_colsum<T>, dim3((unsigned)((n + 63) / 64 * (long)B)), dim3(256), 0, st, X, starts, S, n, (T*)ws);
+  MITOK_LAUNCH(k_seq_sum<T>, dim3((n + 255) / 256), dim3(256), 0, st, (const T*)ws, B, n, mult, out);
 }
-
-void bias_grad(hipStream_t st, const double2* G, int B, int S, int V, double2* ws, double2* db) {
-  colsum(st, G, B, S, V, 1.0, ws, db);
+void colsum(hipStream_t st, const double2* X, int B, int S, int n, double mult, double2* ws, double2* out) {
+  colsum_of(st, X, nullptr, B, S, n, mult, ws, out);
+}
+void colsum_packed(hipStream_t st, const double* X, const int* starts, int B, int n, double2* ws, double2* out) {
+  colsum_of(st, X, starts, B, 0, n, 1.0, ws, out);
 }
 
 void linear_update(hipStream_t st, double2* W, const double2* dW, double2* mW, double2* vW, long n, double2* b,
@@ -260,18 +301,6 @@ __device__ double2 block_sum2(double2 v, double2* sh) {
   __syncthreads();
   return r;
 }
-__device__ double block_max1(double v, double* sh) {
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + w]);
-    __syncthreads();
-  }
-  const double r = sh[0];
-  __syncthreads();
-  return r;
-}
-
 // f64 / Complex and Complex::powf (num-complex 0.4.6: from_polar(r^e, theta e))
 __device__ __forceinline__ double2 rdivc(double a, double2 z) {
   const double ns = z.x * z.x + z.y * z.y;
@@ -351,113 +380,70 @@ __global__ __launch_bounds__(256) void k_norm_backward(const double2* __restrict
 }
 
 
-// One query row of one head (grid: S x H x B): the forward's attention
-// weights A (masked_attention_head.rs:184-205: Re of the scaled scores plus
-// Re(bias_pos), the causal mask, softmax_complex_padding_real) and
-// dl_da = backpropagate_softmax_masked_real of dl_ds = G conj(V)^T over the
-// row Jacobian s_j (delta_jk - s_k) (utils/derivative.rs:100-131, 253-272):
-// dA_j = s_j (r_j - sum_k s_k r_k), r_k = Re(dl_ds_k); padded rows 0.
-__global__ __launch_bounds__(256) void k_attn_probs_grad(const double2* __restrict__ qkv, const double* __restrict__ bias_re,
-                                                         int mc, const uint32_t* __restrict__ mask,
-                                                         const double2* __restrict__ G, int S, int H, int dh, double c,
-                                                         double* __restrict__ A, double* __restrict__ dA) {
-  extern __shared__ double dyn[];
-  double* sc = dyn;       // [S] scores, then weights
-  double* rr = dyn + S;   // [S] Re(dl_ds)
-  __shared__ double2 qs[256], gs[256];  // the row's q and gradient (dh <= 256)
-  __shared__ double shm[256];
-  __shared__ double2 sh2[256];
-  const int i = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
-  const int d = H * dh, ld = 3 * d;
-  const long row = (long)b * S + i;
-  double* Ar = A + (((long)b * H + h) * S + i) * S;
-  double* dAr = dA + (((long)b * H + h) * S + i) * S;
-  if (mask[row] == 0) {
-    for (int j = tid; j < S; j += 256) Ar[j] = dAr[j] = 0.0;
+// The attention weights and their gradient from two products' results, one
+// wave per query row of a head: A holds Re(q.k) (masked_attention_head.rs:
+// 184-205: scaled, plus Re(bias_pos), the causal mask) and becomes
+// softmax_complex_padding_real's weights s; dA holds r = Re(dl_ds), dl_ds = G
+// conj(V)^T, and becomes backpropagate_softmax_masked_real over the row
+// Jacobian s_j (delta_jk - s_k) (utils/derivative.rs:100-131, 253-272):
+// dA_j = s_j (r_j - sum_k s_k r_k).  Padded rows 0.  NPL values of a row per
+// lane, so both arrays are read and written once.  With the products on the
+// matrix cores (8 x 8 heads of 128 rows): 10 us beside 26 us of products, where
+// one block per row formed its own dot products in 97.
+template <int NPL>
+__global__ __launch_bounds__(256) void k_attn_probs_grad(double* __restrict__ A, double* __restrict__ dA,
+                                                         const double* __restrict__ bias_re, int mc,
+                                                         const uint32_t* __restrict__ mask, long rows, int S, int H,
+                                                         double c) {
+  const int lane = threadIdx.x & 63;
+  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int i = (int)(row % S), h = (int)(row / S % H);
+  const long b = row / S / H;
+  double* a = A + row * S;
+  double* g = dA + row * S;
+  if (mask[b * S + i] == 0) {
+    for (int j = lane; j < S; j += 64) a[j] = g[j] = 0.0;
     return;
   }
-  for (int m = tid; m < dh; m += 256) {
-    qs[m] = qkv[row * ld + (long)h * dh + m];
-    gs[m] = G[row * d + (long)h * dh + m];
-  }
-  __syncthreads();
-  // 16 lanes per key (a key's row read in contiguous 16-lane runs), 16 keys per pass
   const double* bp = bias_re + ((long)h * mc + i) * mc;
-  const int sub = tid & 15, kq = tid >> 4;
-  for (int j0 = 0; j0 < S; j0 += 16) {
-    const int j = j0 + kq;
-    double s = 0.0, rv = 0.0;
-    if (j < S) {
-      const double2* k = qkv + ((long)b * S + j) * ld + d + (long)h * dh;
-      const double2* v = k + d;
-      for (int m = sub; m < dh; m += 16) {
-        const double2 kk = k[m], vv = v[m];
-        s = s + (qs[m].x * kk.x - qs[m].y * kk.y);
-        rv = rv + (gs[m].x * vv.x + gs[m].y * vv.y);
-      }
-    }
-    s = row16_sum(s);
-    rv = row16_sum(rv);
-    if (j < S && sub == 0) {
-      sc[j] = j > i ? -1e12 : s * c + bp[j];
-      rr[j] = rv;
-    }
-  }
-  __syncthreads();
+  double sc[NPL], rr[NPL];
   double mx = -INFINITY;
-  for (int j = tid; j < S; j += 256) mx = fmax(mx, sc[j]);
-  mx = block_max1(mx, shm);
-  double2 acc = make_double2(0.0, 0.0);
-  for (int j = tid; j < S; j += 256) {
-    sc[j] = exp(sc[j] - mx);
-    acc.x += sc[j];
+#pragma unroll
+  for (int t = 0; t < NPL; ++t) {
+    const int j = lane + 64 * t;
+    sc[t] = -INFINITY, rr[t] = 0.0;
+    if (j < S) {
+      sc[t] = j > i ? -1e12 : a[j] * c + bp[j];
+      rr[t] = g[j];
+    }
+    mx = fmax(mx, sc[t]);
   }
-  const double sum = block_sum2(acc, sh2).x;
-  acc = make_double2(0.0, 0.0);
-  for (int j = tid; j < S; j += 256) {
-    sc[j] = sc[j] / sum;
-    acc.x += sc[j] * rr[j];
+  mx = wave_max(mx);
+  double sum = 0.0;
+#pragma unroll
+  for (int t = 0; t < NPL; ++t)
+    if (lane + 64 * t < S) {
+      sc[t] = exp(sc[t] - mx);
+      sum += sc[t];
+    }
+  sum = wave_sum(sum);
+  double sr = 0.0;
+#pragma unroll
+  for (int t = 0; t < NPL; ++t)
+    if (lane + 64 * t < S) {
+      sc[t] = sc[t] / sum;
+      sr += sc[t] * rr[t];
+    }
+  sr = wave_sum(sr);
+#pragma unroll
+  for (int t = 0; t < NPL; ++t) {
+    const int j = lane + 64 * t;
+    if (j < S) {
+      a[j] = sc[t];
+      g[j] = sc[t] * (rr[t] - sr);
+    }
   }
-  const double sr = block_sum2(acc, sh2).x;
-  for (int j = tid; j < S; j += 256) {
-    Ar[j] = sc[j];
-    dAr[j] = sc[j] * (rr[j] - sr);
-  }
-}
-
-// The three small products of MaskedAttentionHead::backward per (sequence,
-// head), one output element each (masked_attention_head.rs:276-316):
-//   dV = A^T G,  dQ = dA conj(K) c,  dK = dA^T conj(Q) c
-// written as the gradient of the packed [q | k | v] row (head h at h*dh).
-__global__ __launch_bounds__(256) void k_attn_dqkv(const double2* __restrict__ qkv, const double* __restrict__ A,
-                                                   const double* __restrict__ dA, const double2* __restrict__ G, int B,
-                                                   int S, int H, int dh, double c, double2* __restrict__ dqkv) {
-  const long t = (long)blockIdx.x * 256 + threadIdx.x;
-  const long total = (long)B * H * S * dh;
-  if (t >= total) return;
-  const int m = (int)(t % dh);
-  const int i = (int)((t / dh) % S);
-  const int h = (int)((t / ((long)dh * S)) % H);
-  const int b = (int)(t / ((long)dh * S * H));
-  const int d = H * dh, ld = 3 * d;
-  const double* Ab = A + ((long)b * H + h) * S * S;
-  const double* dAb = dA + ((long)b * H + h) * S * S;
-  const double2* base = qkv + (long)b * S * ld + (long)h * dh + m;
-  const double2* gb = G + (long)b * S * d + (long)h * dh + m;
-  double2 dq = make_double2(0.0, 0.0), dk = dq, dv = dq;
-  for (int j = 0; j < S; ++j) {
-    const double2 kj = base[(long)j * ld + d];     // K[j][m]
-    const double2 qj = base[(long)j * ld];         // Q[j][m]
-    const double a = dAb[(long)i * S + j];         // dA[i][j]
-    const double at = dAb[(long)j * S + i];        // dA[j][i]
-    dq = cadd(dq, make_double2(a * kj.x, -a * kj.y));
-    dk = cadd(dk, make_double2(at * qj.x, -at * qj.y));
-    dv = cadd(dv, cscale(gb[(long)j * d], Ab[(long)j * S + i]));
-  }
-  double2* o = dqkv + ((long)b * S + i) * ld + (long)h * dh + m;
-  o[0] = cscale(dq, c);
-  o[d] = cscale(dk, c);
-  o[2 * d] = dv;
 }
 
 // bias_pos's update on its S x S slice (masked_attention_head.rs:387-393,
@@ -549,23 +535,14 @@ void norm_backward(hipStream_t st, const double2* x, const double2* resid, long 
   if (rows > 0) MITOK_LAUNCH(k_norm_backward, dim3((unsigned)rows), dim3(256), 0, st, x, resid, n, eps, gamma, beta, dout, dx, pg);
 }
 
-void colsum(hipStream_t st, const double2* X, int B, int S, int n, double mult, double2* ws, double2* out) {
-  if (n <= 0 || B <= 0) return;
-  MITOK_LAUNCH(k_seq_colsum, dim3((unsigned)(((long)B * n + 255) / 256)), dim3(256), 0, st, X, B, S, n, ws);
-  MITOK_LAUNCH(k_seq_sum, dim3((n + 255) / 256), dim3(256), 0, st, ws, B, n, mult, out);
-}
-
-void attn_probs_grad(hipStream_t st, const double2* qkv, const double* bias_re, int mc, const uint32_t* mask,
-                     const double2* G, int B, int S, int H, int dh, double c, double* A, double* dA) {
-  MITOK_LAUNCH(k_attn_probs_grad, dim3(S, H, B), dim3(256), (size_t)2 * S * sizeof(double), st, qkv, bias_re, mc, mask,
-               G, S, H, dh, c, A, dA);
-}
-
-void attn_dqkv(hipStream_t st, const double2* qkv, const double* A, const double* dA, const double2* G, int B, int S,
-               int H, int dh, double c, double2* dqkv) {
-  const long total = (long)B * H * S * dh;
-  if (total > 0)
-    MITOK_LAUNCH(k_attn_dqkv, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, qkv, A, dA, G, B, S, H, dh, c, dqkv);
+void attn_probs_grad(hipStream_t st, double* A, double* dA, const double* bias_re, int mc, const uint32_t* mask, int B,
+                     int S, int H, double c) {
+  const long rows = (long)B * H * S;
+  const dim3 grid((unsigned)((rows + 3) / 4)), blk(256);
+  if (rows <= 0) return;
+  if (S <= 64 * 2) MITOK_LAUNCH(k_attn_probs_grad<2>, grid, blk, 0, st, A, dA, bias_re, mc, mask, rows, S, H, c);
+  else if (S <= 64 * 8) MITOK_LAUNCH(k_attn_probs_grad<8>, grid, blk, 0, st, A, dA, bias_re, mc, mask, rows, S, H, c);
+  else MITOK_LAUNCH(k_attn_probs_grad<48>, grid, blk, 0, st, A, dA, bias_re, mc, mask, rows, S, H, c);  // S <= 3072
 }
 
 void attn_bias_update(hipStream_t st, double* bias_re, int mc, const double* dA, int B, int H, int S, const TrainStep& ts) {

@@ -32,6 +32,9 @@ struct MfmaBatch {
   int n = 1, inner = 1;
   long a0 = 0, a1 = 0, b0 = 0, b1 = 0, c0 = 0, c1 = 0;
   double scale = 1.0;
+  // a real A: the row a zero row of A would give, [N], zeros before the launch;
+  // NaN is left where B's column holds an infinity or NaN
+  double2* zero_row = nullptr;
 };
 // ERR_ARG for a combination of mode and operand forms nothing uses
 int launch_zgemm_mfma(hipStream_t st, const MfmaPlan& p, const GemmOpnd& A, const GemmOpnd& B, int M, int N, int K,
@@ -51,9 +54,13 @@ struct TrainStep {
   double batch = 1;   // sequences in the batch (the descent divides by it)
   int time_step = 0;  // AdamW's bias-correction step (at least 1)
 };
-// G[r][c] (complex, im 0) = tgt[r] < 0 ? 0 : (P[r][c] - [c == tgt[r]]) / norm[r / S]
-void softmax_grad(hipStream_t st, const double* P, int rows, int V, const int* tgt, const double* norm, int S,
-                  double2* G);
+// packed softmax gradient G [n][V]: row i = (P[r][c] - [c == tgt[r]]) / norm[r / S] of r = rows[i], zeros for r < 0
+void softmax_grad(hipStream_t st, const double* P, int n, int V, const int* rows, const int* tgt, const double* norm,
+                  int S, double* G);
+// out[packed[r]] = X[r]; the rows of packed row `zero` leave zeros there, NaN where one of them is not finite
+void pack_rows(hipStream_t st, const double2* X, long rows, int d, const int* packed, int zero, double2* out);
+// out[r] = in[packed[r]]
+void unpack_rows(hipStream_t st, const double2* in, long rows, int d, const int* packed, double2* out);
 // cross_entropy_loss_batch of P [B][S][V] for targets [B][T] (tlen[b] each):
 // part [B] the sequences' losses, out [2] the batch loss (re, im); T <= CE_MAX_T
 constexpr int CE_MAX_T = 8192;
@@ -62,25 +69,19 @@ void cross_entropy(hipStream_t st, const double* P, int B, int S, int V, const u
 // G = mask[r] ? dH * conj(GELU'(Z)) : 0 (layer.rs:181-192, derivative.rs:48-84); mask may be null (all rows)
 void gelu_backward(hipStream_t st, const double2* dH, const double2* Z, const uint32_t* mask, long rows, int F,
                    double2* G);
-// out [C][R] = conj(in)^T for in [R][C]
-void conj_transpose(hipStream_t st, const double2* in, long R, long C, double2* out);
-// db [V] = sum_b sum_s G[b][s][:] (per-sequence sums in row order, then in sequence order); ws [B][V]
-void bias_grad(hipStream_t st, const double2* G, int B, int S, int V, double2* ws, double2* db);
 // W [n], b [V] updated in place from dW, db (moments mW, vW, mb, vb)
 void linear_update(hipStream_t st, double2* W, const double2* dW, double2* mW, double2* vW, long n, double2* b,
                    const double2* db, double2* mb, double2* vb, int V, const TrainStep& ts);
 // the Norm's backward per row of x (or Re(x + resid) + 0i); dx real rows, pg = dout * x_hat
 void norm_backward(hipStream_t st, const double2* x, const double2* resid, long rows, int n, double eps,
                    const double2* gamma, const double2* beta, const double2* dout, double2* dx, double2* pg);
-// out[j] = mult * (sum over sequences b of the row sum of X[b][:][j]), as bias_grad; ws [B][n]
+// out[j] = mult * sum over sequences b of the row sum of X[b][:][j] (rows in order, then sequences); ws [B][n]
 void colsum(hipStream_t st, const double2* X, int B, int S, int n, double mult, double2* ws, double2* out);
-// attention weights A and dl_da [B][H][S][S] of a stateless pass from the packed [q | k | v] rows and the
-// gradient G [B*S][d] of the heads' output
-void attn_probs_grad(hipStream_t st, const double2* qkv, const double* bias_re, int mc, const uint32_t* mask,
-                     const double2* G, int B, int S, int H, int dh, double c, double* A, double* dA);
-// the gradient of the packed [q | k | v] rows: dQ = c dA conj(K), dK = c dA^T conj(Q), dV = A^T G
-void attn_dqkv(hipStream_t st, const double2* qkv, const double* A, const double* dA, const double2* G, int B, int S,
-               int H, int dh, double c, double2* dqkv);
+// the same of packed real rows, sequence b's at [starts[b], starts[b + 1])
+void colsum_packed(hipStream_t st, const double* X, const int* starts, int B, int n, double2* ws, double2* out);
+// A [B][H][S][S]: Re(q.k) in, attention weights out; dA: Re(G conj(V)^T) in, dl_da out (S <= 3072)
+void attn_probs_grad(hipStream_t st, double* A, double* dA, const double* bias_re, int mc, const uint32_t* mask, int B,
+                     int S, int H, double c);
 // Re(bias_pos)[h][:S][:S] updated from dA summed over the batch (zero moments each call)
 void attn_bias_update(hipStream_t st, double* bias_re, int mc, const double* dA, int B, int H, int S,
                       const TrainStep& ts);
