@@ -295,6 +295,7 @@ struct Spec {
   bool compress = false;             // apply the wavelet stages begin_call planned for this call
   double* hist_re = nullptr;         // Re-logits history [step][B][V] at hist_cnt[0] (token loop)
   const int* hist_cnt = nullptr;
+  int S_out = 0;                     // sizing: rows per sequence after a compression (0: S)
   int ctx_bound = 0;                 // keys a decode step of this call can reach (0: the layers' context)
 };
 
@@ -393,6 +394,13 @@ struct mitok_network {
   // the heads' output of each SelfAttention layer (before its residual + Norm)
   std::vector<std::unique_ptr<mitok::DevBuf>> tr_in, tr_cat;
   std::vector<char> tr_real;  // whether a layer's input rows had zero imaginary parts
+  // the forward products backward reads: a FeedForward's pre-activation and
+  // hidden rows, an attention layer's q rows and its k and v rows.  tr_saved:
+  // the buffers are there (they are left out, and backward forms the products
+  // again, where the device has no room); tr_fresh: they hold the last
+  // stateless pass's values under the weights as they are
+  std::vector<std::unique_ptr<mitok::DevBuf>> sv_a, sv_b;
+  bool tr_saved = false, tr_fresh = false;
   mitok::DevBuf tr_g, tr_xh, tr_dw, tr_db, tr_ga, tr_gb, tr_tgt, tr_norm;
   mitok::DevBuf tr_z, tr_h, tr_g1, tr_dh, tr_qkv, tr_dqkv, tr_A, tr_dA, tr_pg, tr_eid, tr_est, tr_eocc, tr_bsum;
   mitok::DevBuf ce_buf;  // mitok_cross_entropy_loss: targets, lengths, per-sequence losses, the result
@@ -557,6 +565,30 @@ static bool is_vocab_linear(const Net* n, uint32_t li) {
   return n->layers[li]->kind == K_LINEAR && li + 2 == n->layers.size() && n->layers.back()->kind == K_SOFTMAX;
 }
 
+// a stateless pass from the Embedding on is what backward may differentiate
+static bool keeps(const Spec& sp) { return sp.mode == MODE_STATELESS && sp.first == 0; }
+
+// Gives up the saved forward products: backward then forms them again.
+static void drop_saved(Net* n) {
+  for (auto* v : {&n->sv_a, &n->sv_b})
+    for (auto& b : *v) b->release();
+  n->tr_saved = n->tr_fresh = false;
+}
+
+// Room for the forward products of `rows` rows (at most) that backward reads
+static int reserve_saved(Net* n, const Spec& sp, size_t rows) {
+  for (auto* v : {&n->sv_a, &n->sv_b})
+    while (v->size() < n->layers.size()) v->push_back(std::make_unique<DevBuf>());
+  for (uint32_t li = sp.first; li < sp.last; ++li) {
+    const Layer* L = n->layers[li].get();
+    const size_t a = L->kind == K_FEED_FORWARD ? ((const FeedForwardLayer*)L)->hidden : L->d_in;
+    if (L->kind != K_FEED_FORWARD && L->kind != K_SELF_ATTENTION) continue;
+    TRY(reserve(n, *n->sv_a[li], rows * a * sizeof(double2)));  // Z | q rows
+    TRY(reserve(n, *n->sv_b[li], rows * (L->kind == K_FEED_FORWARD ? a : 2 * a) * sizeof(double2)));  // H | k, v
+  }
+  return OK;
+}
+
 static int prepare(Net* n, const Spec& sp) {
   n->head_valid = false;  // the workspaces that held the last stateless pass's head input are reused
   const Dims dm = net_dims(n);
@@ -570,7 +602,7 @@ static int prepare(Net* n, const Spec& sp) {
   TRY(reserve(n, n->gath, (size_t)sp.B * dm.dmax * c16));
   TRY(reserve(n, n->mat0, rows * dm.dmax * c16));
   TRY(reserve(n, n->mat1, rows * dm.dmax * c16));
-  if (sp.mode == MODE_STATELESS) {  // the layer inputs backward reads
+  if (keeps(sp)) {  // the layer inputs backward reads
     while (n->tr_in.size() < n->layers.size()) n->tr_in.push_back(std::make_unique<DevBuf>());
     while (n->tr_cat.size() < n->layers.size()) n->tr_cat.push_back(std::make_unique<DevBuf>());
     n->tr_real.assign(n->layers.size(), 0);
@@ -581,19 +613,23 @@ static int prepare(Net* n, const Spec& sp) {
     }
   }
   size_t ws = 0;
+  const auto product = [&](int m, int N, int K) {  // split workspace of a product, before or after a compression
+    ws = std::max(ws, gemm_ws_bytes(m, N, K));
+    if (sp.S_out && m == (int)rows) ws = std::max(ws, gemm_ws_bytes(sp.B * sp.S_out, N, K));
+  };
   for (uint32_t li = sp.first; li < sp.last; ++li) {
     Layer* L = n->layers[li].get();
     const int M = (int)rows;
-    if (L->kind == K_SELF_ATTENTION) ws = std::max(ws, gemm_ws_bytes(M, 3 * L->d_in, L->d_in));
+    if (L->kind == K_SELF_ATTENTION) product(M, 3 * L->d_in, L->d_in);
     if (L->kind == K_FEED_FORWARD) {
       auto* F = (FeedForwardLayer*)L;
-      ws = std::max(ws, gemm_ws_bytes(M, F->hidden, F->d_in));
-      ws = std::max(ws, gemm_ws_bytes(M, F->d_out, F->hidden));
+      product(M, F->hidden, F->d_in);
+      product(M, F->d_out, F->hidden);
     }
     if (L->kind == K_LINEAR) {
       const bool vocab = is_vocab_linear(n, li) && sp.first == 0;
       const int Mv = (vocab && sp.last_row) ? sp.B : M;
-      ws = std::max(ws, gemm_ws_bytes(Mv, L->d_out, L->d_in));
+      product(Mv, L->d_out, L->d_in);
       if (vocab && !sp.forward_only) {
         TRY(reserve(n, n->probs, (size_t)Mv * L->d_out * sizeof(double)));
       }
@@ -607,7 +643,7 @@ static int prepare(Net* n, const Spec& sp) {
   if (dm.hmax) {
     if (sp.mode == MODE_CACHED && sp.S == 1)
       TRY(reserve(n, n->datt, attention_split_ws_bytes(sp.B, dm.hmax, dm.dh_max, dm.mc_max)));
-    if (sp.mode == MODE_STATELESS) TRY(reserve(n, n->kv_scratch, 2 * rows * dm.dsa * c16));
+    if (sp.mode == MODE_STATELESS && !keeps(sp)) TRY(reserve(n, n->kv_scratch, 2 * rows * dm.dsa * c16));
   }
   TRY(reserve(n, n->sync_ws, ws));
   if (sp.mode == MODE_CACHED && sp.S == 1 && sp.B <= GEMM_PART_MAX_M) {
@@ -621,6 +657,14 @@ static int prepare(Net* n, const Spec& sp) {
   if (n->pos_off) TRY(reserve(n, n->pos_off_d, (size_t)sp.B * sizeof(int)));
   TRY(reserve(n, n->ones_d, std::max<size_t>(rows, sp.B) * sizeof(uint32_t)));
   TRY(reserve(n, n->dec_ids_d, (size_t)sp.B * sizeof(uint32_t)));
+  if (keeps(sp)) {
+    n->tr_fresh = false;
+    n->tr_saved = reserve_saved(n, sp, rows) == OK;
+    if (!n->tr_saved) {  // no room: the pass itself needs only this
+      drop_saved(n);
+      if (dm.hmax) TRY(reserve(n, n->kv_scratch, 2 * rows * dm.dsa * c16));
+    }
+  }
   return OK;
 }
 
@@ -686,23 +730,38 @@ static int enqueue_forward(Net* n, const Spec& sp) {
   const int* pos = sp.pos;
   size_t wi = 0;  // next wavelet stage
   bool real = false;  // the rows in cur have zero imaginary parts: a Norm leaves Re(x) + 0i (norm_layer.rs:64-130)
+  // a pass that backward may differentiate leaves every layer's input in that
+  // layer's own buffer; another alternates between two
+  const bool keep = keeps(sp), save = keep && n->tr_saved;
+  const auto keeps_input = [&](uint32_t li) {
+    return keep && li < sp.last && n->layers[li]->kind != K_EMBEDDING && n->layers[li]->kind != K_SOFTMAX;
+  };
   double2* cur = n->act0.as<double2>();
   double2* nxt = n->act1.as<double2>();
+  if (keep) n->tr_fresh = save;
   if (sp.in) HIP_TRY(hipMemcpyAsync(cur, sp.in, (size_t)rows * n->layers[sp.first]->d_in * sizeof(double2),
                                    hipMemcpyDeviceToDevice, st));
   for (uint32_t li = sp.first; li < sp.last; ++li) {
     Layer* L = n->layers[li].get();
-    if (sp.mode == MODE_STATELESS && L->kind != K_EMBEDDING && L->kind != K_SOFTMAX)  // kept for backward
-      HIP_TRY(hipMemcpyAsync(n->tr_in[li]->p, cur, (size_t)rows * L->d_in * sizeof(double2), hipMemcpyDeviceToDevice, st));
-    if (sp.mode == MODE_STATELESS) n->tr_real[li] = real;
+    if (keep) n->tr_real[li] = real;
+    nxt = keeps_input(li + 1) ? n->tr_in[li + 1]->as<double2>()
+                              : cur == n->act0.as<double2>() ? n->act1.as<double2>() : n->act0.as<double2>();
+    const auto pass_on = [&]() -> int {  // the layer works in place, or not at all
+      if (!keeps_input(li + 1)) return OK;
+      HIP_TRY(hipMemcpyAsync(nxt, cur, (size_t)rows * L->d_out * sizeof(double2), hipMemcpyDeviceToDevice, st));
+      cur = nxt;
+      return OK;
+    };
     switch (L->kind) {
       case K_EMBEDDING: {
         auto* E = (EmbeddingLayer*)L;
-        embed(st, E->table.as<double2>(), E->vocab, E->d_out, sp.ids, rows, cur, err);
+        embed(st, E->table.as<double2>(), E->vocab, E->d_out, sp.ids, rows, nxt, err);
+        cur = nxt;
         break;
       }
       case K_POSENC: {
         auto* P = (PositionalEncodingLayer*)L;
+        TRY(pass_on());
         rope(st, cur, rows, P->d_in, P->cs.as<double2>(), P->positions, pos, pos ? nullptr : n->kv_len_d.as<int>(),
              pos ? nullptr : rope_offsets(n), err);
         break;
@@ -710,7 +769,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
       case K_NORM: {
         auto* N = (NormLayer*)L;
         layernorm(st, cur, nullptr, nxt, rows, N->d_in, N->eps, N->gamma.as<double2>(), N->beta.as<double2>());
-        std::swap(cur, nxt);
+        cur = nxt;
         real = true;
         break;
       }
@@ -719,7 +778,9 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         const int d = A->d_in, H = A->heads, dh = A->dh;
         Epi e;
         e.mode = EPI_QKV;
-        e.out = n->qbuf.as<double2>();
+        double2* q = save ? n->sv_a[li]->as<double2>() : n->qbuf.as<double2>();
+        double2* cat = keep ? n->tr_cat[li]->as<double2>() : n->concat.as<double2>();
+        e.out = q;
         e.ldo = d;
         e.d = d;
         e.dh = dh;
@@ -727,10 +788,10 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         e.S = S;
         e.err = err;
         Attn a;
-        a.q = n->qbuf.as<double2>();
+        a.q = q;
         a.ldq = d;
         if (sp.mode == MODE_STATELESS) {
-          e.kc = n->kv_scratch.as<double2>();
+          e.kc = save ? n->sv_b[li]->as<double2>() : n->kv_scratch.as<double2>();
           e.vc = e.kc + (size_t)rows * d;
           e.ctx = S;
           a.T_const = S;
@@ -761,7 +822,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         a.bias_re = A->bias_re.as<double>();
         a.mc = A->max_ctx;
         a.row_mask = mask;
-        a.out = n->concat.as<double2>();
+        a.out = cat;
         a.ldo = d;
         a.B = B;
         a.S = S;
@@ -790,13 +851,10 @@ static int enqueue_forward(Net* n, const Spec& sp) {
             TimeScope ts(n, MITOK_TIME_ATTENTION, 0.0);
             if (!n->tiled_prefill || !attention_prefill(st, a)) attention_rows(st, a);
           }
-          if (sp.mode == MODE_STATELESS)  // the heads' output, kept for backward
-            HIP_TRY(hipMemcpyAsync(n->tr_cat[li]->p, n->concat.p, (size_t)rows * d * sizeof(double2),
-                                   hipMemcpyDeviceToDevice, st));
-          layernorm(st, n->concat.as<double2>(), cur, nxt, rows, d, A->eps, A->gamma.as<double2>(),
+          layernorm(st, cat, cur, nxt, rows, d, A->eps, A->gamma.as<double2>(),
                     A->beta.as<double2>());
         }
-        std::swap(cur, nxt);
+        cur = nxt;
         real = true;
         break;
       }
@@ -805,7 +863,9 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         Epi e1;
         e1.mode = EPI_GELU;
         e1.bias = F->b1.as<double2>();
-        e1.out = n->hbuf.as<double2>();
+        double2* h = save ? n->sv_b[li]->as<double2>() : n->hbuf.as<double2>();
+        e1.out = h;
+        e1.pre = save ? n->sv_a[li]->as<double2>() : nullptr;
         e1.ldo = F->hidden;
         e1.row_mask = mask;
         e1.err = err;
@@ -825,10 +885,10 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         {
           TimeScope ts(n, S > 1 ? MITOK_TIME_PREFILL_GEMM : MITOK_TIME_LAYER_GEMM, gemm_bytes(rows, F->d_out, F->hidden, false),
                        gemm_flops(rows, F->d_out, F->hidden));
-          TRY(launch_rc(gemm(st, rows, F->d_out, F->hidden, rows_of(n->hbuf.as<double2>(), F->hidden),
+          TRY(launch_rc(gemm(st, rows, F->d_out, F->hidden, rows_of(h, F->hidden),
                              F->w2.as<double2>(), F->d_out, e2, nullptr, sy), "ffn2"));
         }
-        std::swap(cur, nxt);
+        cur = nxt;
         real = false;
         break;
       }
@@ -844,7 +904,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
           e.err = err;
           TRY(launch_rc(gemm(st, rows, Ln->d_out, Ln->d_in, rows_of(cur, Ln->d_in, real), Ln->w.as<double2>(), Ln->d_out, e,
                              nullptr, sy), "linear"));
-          std::swap(cur, nxt);
+          cur = nxt;
           real = false;
           break;
         }
@@ -891,11 +951,14 @@ static int enqueue_forward(Net* n, const Spec& sp) {
       case K_WAVELET: {
         // only the call begin_call planned compresses; a cached step's row
         // passes through (wavelet_discrete_layer.rs:102-128)
-        if (!sp.compress) break;
+        if (!sp.compress) {
+          TRY(pass_on());
+          break;
+        }
         if (wi >= n->wstages.size()) return fail(ERR_STATE, "wavelet stage %zu not planned", wi);
         const auto& W = *n->wstages[wi++];
         dwt_rows(st, cur, B, S, (int)L->d_in, W.src.as<int>(), W.sgn.as<double>(), W.lo_d.as<double>(), W.L, W.S2, nxt);
-        std::swap(cur, nxt);
+        cur = nxt;
         S = W.S2;
         rows = B * S;
         mask = W.mask.as<uint32_t>();
@@ -1950,6 +2013,7 @@ int mitok_init_seeded(mitok_network* n, uint64_t seed) {
   if (!n) return fail(ERR_ARG, "null network");
   TRY(set_device(n));
   hipStream_t st = n->stream;
+  n->tr_fresh = false;  // the saved forward products are of other weights
   auto lim = [](uint64_t r, uint64_t c) { return sqrt(6.0 / (double)(r + c)); };
   for (uint32_t li = 0; li < n->layers.size(); ++li) {
     Layer* L = n->layers[li].get();
@@ -2142,6 +2206,7 @@ static int begin_call(Net* n, const uint32_t* lens, uint32_t B, uint32_t S, cons
   if (mc != UINT32_MAX && (uint32_t)Sc > mc) return fail(ERR_ARG, "sequence %d exceeds max context %u", Sc, mc);
   Spec sz = sp;
   sz.S = S_alloc;
+  sz.S_out = wl.empty() ? 0 : Sc;
   TRY(prepare(n, sz));
   if (sp.mode == MODE_PREFILL) TRY(alloc_caches(n, B));
   const size_t rows = (size_t)B * S;
@@ -2779,7 +2844,7 @@ int mitok_decode_step(mitok_network* n, const uint32_t* ids, uint32_t B, uint32_
 // the AdamW moments of a weight (nw) and its bias (nb), allocated and zeroed
 // at the first update; nb = 0: a lone array's pair (mw, vw) only
 static int ensure_moments(hipStream_t st, size_t nw, size_t nb, DevBuf& mw, DevBuf& vw, DevBuf& mb, DevBuf& vb) {
-  if (mw.p) return OK;
+  if (mw.p && vw.p && (!nb || (mb.p && vb.p))) return OK;
   TRY(mw.reserve(nw * sizeof(double2)));
   TRY(vw.reserve(nw * sizeof(double2)));
   fill_const(st, mw.as<double2>(), nw, make_double2(0.0, 0.0));
@@ -2996,52 +3061,64 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
     TRY(upload(n, W.gw, keep_d.back().data(), keep_d.back().size() * sizeof(double)));
   }
   // every workspace is sized before the first launch (a reserve that grows frees the old buffer)
-  TRY(upload(n, n->tr_tgt, head.data(), head.size() * sizeof(int)));
-  TRY(upload(n, n->tr_norm, norm.data(), norm.size() * sizeof(double)));
-  if (embed_upd && !eids.empty()) {
-    TRY(upload(n, n->tr_eid, eids.data(), eids.size() * sizeof(uint32_t)));
-    TRY(upload(n, n->tr_est, estart.data(), estart.size() * sizeof(int)));
-    TRY(upload(n, n->tr_eocc, eocc.data(), eocc.size() * sizeof(int)));
-  }
-  TRY(reserve(n, n->tr_g, (size_t)packed * V * sizeof(double)));
-  TRY(reserve(n, n->tr_ga, (size_t)rows_max * dmax * c16));
-  TRY(reserve(n, n->tr_gb, (size_t)rows_max * dmax * c16));
-  TRY(reserve(n, n->tr_xh, (size_t)2 * packed * d * c16));  // packed head input, packed input gradient
-  TRY(reserve(n, n->tr_dw, wmax * c16));
-  TRY(reserve(n, n->tr_db, std::max(bmax, dmax) * c16));
-  TRY(reserve(n, n->tr_dh, (size_t)rows_max * std::max(fmax, dmax) * c16));
-  TRY(reserve(n, n->tr_pg, (size_t)rows_max * dmax * c16));
-  TRY(reserve(n, n->tr_bsum, (size_t)B * std::max({bmax, dmax, fmax}) * c16));  // per-sequence column sums
-  if (fmax) {
-    TRY(reserve(n, n->tr_z, (size_t)rows_max * fmax * c16));
-    TRY(reserve(n, n->tr_h, (size_t)rows_max * fmax * c16));
-    TRY(reserve(n, n->tr_g1, (size_t)rows_max * fmax * c16));
-  }
-  if (att) {
-    TRY(reserve(n, n->tr_qkv, (size_t)rows_max * d3max * c16));
-    TRY(reserve(n, n->tr_dqkv, (size_t)rows_max * d3max * c16));
-    TRY(reserve(n, n->tr_A, (size_t)B * att * sizeof(double)));
-    TRY(reserve(n, n->tr_dA, (size_t)B * att * sizeof(double)));
-  }
-  TRY(reserve(n, n->sync_ws, ws));
-  if (update_params) {  // AdamW moments, zeroed at a layer's first update
-    TRY(ensure_moments(st, (size_t)d * V, V, Ln->mw, Ln->vw, Ln->mb, Ln->vb));
-    for (uint32_t li = stop; li < li_top; ++li) {
-      Layer* L = n->layers[li].get();
-      if (L->kind == K_LINEAR) {
-        auto* H = (LinearLayer*)L;
-        TRY(ensure_moments(st, (size_t)H->d_in * H->d_out, H->d_out, H->mw, H->vw, H->mb, H->vb));
-      } else if (L->kind == K_FEED_FORWARD) {
-        auto* F = (FeedForwardLayer*)L;
-        TRY(ensure_moments(st, (size_t)F->hidden * F->d_out, F->d_out, F->mw2, F->vw2, F->mb2, F->vb2));
-        TRY(ensure_moments(st, (size_t)F->d_in * F->hidden, F->hidden, F->mw1, F->vw1, F->mb1, F->vb1));
-      } else if (L->kind == K_SELF_ATTENTION) {
-        auto* A = (SelfAttentionLayer*)L;
-        TRY(ensure_moments(st, (size_t)3 * A->d_in * A->d_in, A->d_in, A->mw, A->vw, A->mg, A->vg));
-        TRY(ensure_moments(st, A->d_in, 0, A->mbt, A->vbt, A->mbt, A->vbt));
+  const auto size_all = [&]() -> int {
+    TRY(upload(n, n->tr_tgt, head.data(), head.size() * sizeof(int)));
+    TRY(upload(n, n->tr_norm, norm.data(), norm.size() * sizeof(double)));
+    if (embed_upd && !eids.empty()) {
+      TRY(upload(n, n->tr_eid, eids.data(), eids.size() * sizeof(uint32_t)));
+      TRY(upload(n, n->tr_est, estart.data(), estart.size() * sizeof(int)));
+      TRY(upload(n, n->tr_eocc, eocc.data(), eocc.size() * sizeof(int)));
+    }
+    TRY(reserve(n, n->tr_g, (size_t)packed * V * sizeof(double)));
+    TRY(reserve(n, n->tr_ga, (size_t)rows_max * dmax * c16));
+    TRY(reserve(n, n->tr_gb, (size_t)rows_max * dmax * c16));
+    TRY(reserve(n, n->tr_xh, (size_t)2 * packed * d * c16));  // packed head input, packed input gradient
+    TRY(reserve(n, n->tr_dw, wmax * c16));
+    TRY(reserve(n, n->tr_db, std::max(bmax, dmax) * c16));
+    TRY(reserve(n, n->tr_dh, (size_t)rows_max * std::max(fmax, dmax) * c16));
+    TRY(reserve(n, n->tr_pg, (size_t)rows_max * dmax * c16));
+    TRY(reserve(n, n->tr_bsum, (size_t)B * std::max({bmax, dmax, fmax}) * c16));  // per-sequence column sums
+    if (fmax) {
+      if (!n->tr_saved) {
+        TRY(reserve(n, n->tr_z, (size_t)rows_max * fmax * c16));
+        TRY(reserve(n, n->tr_h, (size_t)rows_max * fmax * c16));
+      }
+      TRY(reserve(n, n->tr_g1, (size_t)rows_max * fmax * c16));
+    }
+    if (att) {
+      if (!n->tr_saved) TRY(reserve(n, n->tr_qkv, (size_t)rows_max * d3max * c16));
+      TRY(reserve(n, n->tr_dqkv, (size_t)rows_max * d3max * c16));
+      TRY(reserve(n, n->tr_A, (size_t)B * att * sizeof(double)));
+      TRY(reserve(n, n->tr_dA, (size_t)B * att * sizeof(double)));
+    }
+    TRY(reserve(n, n->sync_ws, ws));
+    if (update_params) {  // AdamW moments, zeroed at a layer's first update
+      TRY(ensure_moments(st, (size_t)d * V, V, Ln->mw, Ln->vw, Ln->mb, Ln->vb));
+      for (uint32_t li = stop; li < li_top; ++li) {
+        Layer* L = n->layers[li].get();
+        if (L->kind == K_LINEAR) {
+          auto* H = (LinearLayer*)L;
+          TRY(ensure_moments(st, (size_t)H->d_in * H->d_out, H->d_out, H->mw, H->vw, H->mb, H->vb));
+        } else if (L->kind == K_FEED_FORWARD) {
+          auto* F = (FeedForwardLayer*)L;
+          TRY(ensure_moments(st, (size_t)F->hidden * F->d_out, F->d_out, F->mw2, F->vw2, F->mb2, F->vb2));
+          TRY(ensure_moments(st, (size_t)F->d_in * F->hidden, F->hidden, F->mw1, F->vw1, F->mb1, F->vb1));
+        } else if (L->kind == K_SELF_ATTENTION) {
+          auto* A = (SelfAttentionLayer*)L;
+          TRY(ensure_moments(st, (size_t)3 * A->d_in * A->d_in, A->d_in, A->mw, A->vw, A->mg, A->vg));
+          TRY(ensure_moments(st, A->d_in, 0, A->mbt, A->vbt, A->mbt, A->vbt));
+        }
       }
     }
+    return OK;
+  };
+  int rc = size_all();
+  if (rc == ERR_NOMEM && n->tr_saved) {  // the forward pass's saved products give way
+    drop_saved(n);
+    rc = size_all();
   }
+  if (rc) return rc;
+  const bool fresh = n->tr_saved && n->tr_fresh;  // the saved forward products are of the weights as they are
   const Sync sy = sync_of(n);
   uint32_t* err = n->err_d.as<uint32_t>();
   long rows_c = rows;  // the current layer's rows (a wavelet layer changes them below it)
@@ -3141,24 +3218,26 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
         // then its Dense (GELU) layer (layer.rs:168-210)
         auto* F = (FeedForwardLayer*)L;
         const int Fh = (int)F->hidden, di = (int)F->d_in, dn = (int)F->d_out;
-        Epi e;
-        e.err = err;
-        e.bias = F->b1.as<double2>();
-        e.ldo = Fh;
-        e.mode = EPI_GELU;  // the Dense output the forward pass gave its Linear: GELU, padded rows 0
-        e.row_mask = mask;
-        e.out = n->tr_h.as<double2>();
-        TRY(launch_rc(gemm(st, (int)rows, Fh, di, rows_of(X, di, xreal), F->w1.as<double2>(), Fh, e, nullptr, sy), "ffn1 output"));
-        e.mode = EPI_STORE;  // its pre-activation Z = X W1 + b1 (layer.rs:135-144)
-        e.row_mask = nullptr;
-        e.out = n->tr_z.as<double2>();
-        TRY(launch_rc(gemm(st, (int)rows, Fh, di, rows_of(X, di, xreal), F->w1.as<double2>(), Fh, e, nullptr, sy),
-                      "ffn1 pre-activation"));
-        TRY(linear_bwd(n->tr_h.as<double2>(), false, gcur, greal, F->w2.as<double2>(), Fh, dn, n->tr_dh.as<double2>()));
+        // the Dense output the forward pass gave its Linear (GELU, padded rows
+        // 0) and its pre-activation Z = X W1 + b1 (layer.rs:135-144)
+        double2* h = n->tr_saved ? n->sv_b[li]->as<double2>() : n->tr_h.as<double2>();
+        double2* z = n->tr_saved ? n->sv_a[li]->as<double2>() : n->tr_z.as<double2>();
+        if (!fresh) {
+          Epi e;
+          e.err = err;
+          e.bias = F->b1.as<double2>();
+          e.ldo = Fh;
+          e.mode = EPI_GELU;
+          e.row_mask = mask;
+          e.out = h;
+          e.pre = z;
+          TRY(launch_rc(gemm(st, (int)rows, Fh, di, rows_of(X, di, xreal), F->w1.as<double2>(), Fh, e, nullptr, sy), "ffn1"));
+        }
+        TRY(linear_bwd(h, false, gcur, greal, F->w2.as<double2>(), Fh, dn, n->tr_dh.as<double2>()));
         // FeedForwardLayer::update_parameters (:219-250): the Linear at the FFN's time step (:86)
         if (update_params) linear_upd(F->w2, F->b2, (long)Fh * dn, dn, F->mw2, F->vw2, F->mb2, F->vb2, F->updates2,
                                       (int)time_step, rate(F));
-        gelu_backward(st, n->tr_dh.as<double2>(), n->tr_z.as<double2>(), mask, rows, Fh, n->tr_g1.as<double2>());
+        gelu_backward(st, n->tr_dh.as<double2>(), z, mask, rows, Fh, n->tr_g1.as<double2>());
         TRY(linear_bwd(X, xreal, n->tr_g1.as<double2>(), false, F->w1.as<double2>(), di, Fh, gnext));
         // the Dense at step 1: Layer::time_step stays 0 after construction (layer.rs:111,285)
         if (update_params) linear_upd(F->w1, F->b1, (long)di * Fh, Fh, F->mw1, F->vw1, F->mb1, F->vb1, F->updates1, 0, rate(F));
@@ -3176,22 +3255,26 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
         double2* gn = n->tr_dh.as<double2>();
         norm_backward(st, n->tr_cat[li]->as<double2>(), X, rows, da, A->eps, A->gamma.as<double2>(), A->beta.as<double2>(),
                       gcur, gn, n->tr_pg.as<double2>());
-        // q rows [rows][da], then k and v as the forward pass holds them, [B][H][S][dh]
-        double2 *q = n->tr_qkv.as<double2>(), *k = q + (size_t)rows * da, *v = k + (size_t)rows * da;
-        Epi e;
-        e.mode = EPI_QKV;
-        e.err = err;
-        e.out = q;
-        e.ldo = da;
-        e.d = da;
-        e.dh = dh;
-        e.heads = H;
-        e.S = S;
-        e.kc = k;
-        e.vc = v;
-        e.ctx = S;
-        TRY(launch_rc(gemm(st, (int)rows, 3 * da, da, rows_of(X, da, xreal), A->wqkv.as<double2>(), 3 * da, e, nullptr, sy),
-                      "qkv"));
+        // q rows [rows][da]; k and v as the forward pass holds them, [B][H][S][dh]
+        double2* q = n->tr_saved ? n->sv_a[li]->as<double2>() : n->tr_qkv.as<double2>();
+        double2* k = n->tr_saved ? n->sv_b[li]->as<double2>() : q + (size_t)rows * da;
+        double2* v = k + (size_t)rows * da;
+        if (!fresh) {
+          Epi e;
+          e.mode = EPI_QKV;
+          e.err = err;
+          e.out = q;
+          e.ldo = da;
+          e.d = da;
+          e.dh = dh;
+          e.heads = H;
+          e.S = S;
+          e.kc = k;
+          e.vc = v;
+          e.ctx = S;
+          TRY(launch_rc(gemm(st, (int)rows, 3 * da, da, rows_of(X, da, xreal), A->wqkv.as<double2>(), 3 * da, e, nullptr, sy),
+                        "qkv"));
+        }
         // the heads' products, one batch entry per (sequence, head): Re(q.k),
         // Re(dl_ds), then dQ = c dA conj(K), dK = c dA^T conj(Q), dV = A^T G
         // (masked_attention_head.rs:276-316) as the gradient of the packed
@@ -3281,7 +3364,10 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
       default: break;
     }
   }
-  if (update_params) drop_graph(n);  // the weights changed under any captured step
+  if (update_params) {
+    drop_graph(n);  // the weights changed under any captured step
+    n->tr_fresh = false;
+  }
   if (out_grad_input) {
     const int dlow = (int)n->layers[stop]->d_in;
     HIP_TRY(hipMemcpyAsync(out_grad_input, gcur, (size_t)rows_c * dlow * c16, hipMemcpyDeviceToHost, st));

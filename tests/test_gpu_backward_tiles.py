@@ -109,3 +109,32 @@ def test_attention_input_gradient(S, d, H, norm):
     gr = oracle.linear_backward(y, oracle.softmax_backward(P, targets), wv)[2]
     want = oracle.self_attention_backward(x, mask, q, k, v, bias, one, nil, gr)[0]
     assert far(dx, want) < TOL
+
+
+def test_second_backward_reads_the_updated_weights():
+    """The forward pass leaves a FeedForward's products for backward; after an
+    update they are formed again from the layer's kept input."""
+    V, d, F, B, S, T = 60, 8, 80, 2, 40, 9
+    r = np.random.default_rng(5)
+    table, w1, b1, w2, b2, wv = c(r, V, d), 0.3 * c(r, d, F), 0.1 * c(r, F), 0.2 * c(r, F, d), 0.1 * c(r, d), 0.1 * c(r, d, V)
+    ids = r.integers(2, V, (B, S)).astype(np.uint32)
+    targets = r.integers(2, V, (B, T)).astype(np.uint32)
+    with ra.Network(0) as net:
+        net.add_embedding(V, d, table)
+        net.add_feed_forward(d, F, w1, b1, w2, b2)
+        net.add_linear(d, V, wv, np.zeros(V, np.complex128))
+        net.add_softmax(ra.TRAINING)
+        P, mask = net.predict(ids, forward_only=False)
+        net.backward(targets, layers=2, update=True, learning_rate=0.5, time_step=1, want_grad_input=False)
+        dx = net.backward(targets, layers=2, update=False)
+        n1, n2, nv = (net.get_tensor(1, 0, d * F).reshape(d, F), net.get_tensor(1, 1, F * d).reshape(F, d),
+                      net.get_tensor(2, 0, d * V).reshape(d, V))
+        nb = net.get_tensor(1, 4, F)
+    assert far(n1, w1) > 1e-4
+    x = table[ids]
+    gelu = np.vectorize(lambda z: oracle.gelu(z)[0])
+    head = gelu(x @ w1 + b1) @ w2 + b2  # the head's input is the forward pass's
+    gr = oracle.linear_backward(head, oracle.softmax_backward(P, targets), nv)[2]
+    z = x @ n1 + nb
+    dh = oracle.linear_backward_c(gelu(z), gr, n2)[2]
+    assert far(dx, oracle.dense_backward(x, z, dh, mask, n1)[2]) < TOL
