@@ -739,15 +739,26 @@ static int enqueue_forward(Net* n, const Spec& sp) {
   double2* cur = n->act0.as<double2>();
   double2* nxt = n->act1.as<double2>();
   if (keep) n->tr_fresh = save;
-  if (sp.in) HIP_TRY(hipMemcpyAsync(cur, sp.in, (size_t)rows * n->layers[sp.first]->d_in * sizeof(double2),
-                                   hipMemcpyDeviceToDevice, st));
+  // a layer range reads the caller's rows and writes the caller's buffer
+  // itself, unless they overlap (no layer writes its input but RoPE, which
+  // copies it)
+  const bool direct = sp.in && sp.out_hidden && [&] {
+    const char *a = (const char*)sp.in, *b = (const char*)sp.out_hidden;
+    const size_t wide = std::max<size_t>(n->layers[sp.first]->d_in, n->layers[sp.last - 1]->d_out) * sizeof(double2);
+    const size_t bytes = (size_t)sp.B * std::max(S, n->wS) * wide;
+    return a + bytes <= b || b + bytes <= a;
+  }();
+  if (direct) cur = const_cast<double2*>(sp.in);
+  else if (sp.in) HIP_TRY(hipMemcpyAsync(cur, sp.in, (size_t)rows * n->layers[sp.first]->d_in * sizeof(double2),
+                                         hipMemcpyDeviceToDevice, st));
   for (uint32_t li = sp.first; li < sp.last; ++li) {
     Layer* L = n->layers[li].get();
     if (keep) n->tr_real[li] = real;
     nxt = keeps_input(li + 1) ? n->tr_in[li + 1]->as<double2>()
                               : cur == n->act0.as<double2>() ? n->act1.as<double2>() : n->act0.as<double2>();
+    if (direct && li + 1 == sp.last) nxt = sp.out_hidden;
     const auto pass_on = [&]() -> int {  // the layer works in place, or not at all
-      if (!keeps_input(li + 1)) return OK;
+      if (!keeps_input(li + 1) && cur != sp.in) return OK;
       HIP_TRY(hipMemcpyAsync(nxt, cur, (size_t)rows * L->d_out * sizeof(double2), hipMemcpyDeviceToDevice, st));
       cur = nxt;
       return OK;
