@@ -101,16 +101,26 @@ __device__ inline double2 csqrt_nc(double2 z) {
     double x = sqrt(fabs(z.y) / 2.0);
     return signbit(z.y) ? make_double2(x, -x) : make_double2(x, x);
   }
-  double r = hypot(z.x, z.y);
-  double th = atan2(z.y, z.x) / 2.0;
-  double rs = sqrt(r);
-  return make_double2(rs * cos(th), rs * sin(th));
+  const double r = hypot(z.x, z.y), rs = sqrt(r);
+  double sn, cs;
+  sincos(atan2(z.y, z.x) / 2.0, &sn, &cs);
+  return make_double2(rs * cs, rs * sn);
 }
-// Complex::tanh: (sinh 2a + i sin 2b) / (cosh 2a + cos 2b)
+// Complex::tanh: (sinh 2a + i sin 2b) / (cosh 2a + cos 2b), sinh and cosh from
+// one u = e^|2a| - 1 (with q = u / (1 + u): (u + q) / 2 and 1 + u q / 2) and
+// one sincos, where four functions each reduced their argument.  cosh + cos,
+// which cancels near a pole, rounds as it did: for GELU of z = 1 + normal of
+// scale 0.1, 0.63, 1 and 3 the rms error is 0.786, 1.007, 74.6 and 266
+// half-ulps, of the four functions 0.817, 1.037, 74.7 and 294 (against 113
+// bits).  FFN Dense, 1024 x 2048 of K 512 on MI355X:
+// 113 -> 101 us.
 __device__ inline double2 ctanh_nc(double2 z) {
-  double a2 = z.x + z.x, b2 = z.y + z.y;
-  double den = cosh(a2) + cos(b2);
-  return make_double2(sinh(a2) / den, sin(b2) / den);
+  const double a2 = z.x + z.x;
+  double s, c;
+  sincos(z.y + z.y, &s, &c);
+  const double u = expm1(fabs(a2)), q = u / (1.0 + u);
+  const double den = fma(0.5 * u, q, 1.0) + c;
+  return make_double2(copysign(0.5 * (u + q), a2) / den, s / den);
 }
 // gelu_complex (utils/activation.rs:195-212); powi(3) = z * (z * z)
 __device__ inline double2 gelu_nc(double2 z, bool* nan) {

@@ -301,14 +301,10 @@ __device__ double2 block_sum2(double2 v, double2* sh) {
   __syncthreads();
   return r;
 }
-// f64 / Complex and Complex::powf (num-complex 0.4.6: from_polar(r^e, theta e))
+// f64 / Complex
 __device__ __forceinline__ double2 rdivc(double a, double2 z) {
   const double ns = z.x * z.x + z.y * z.y;
   return make_double2(a * z.x / ns, -a * z.y / ns);
-}
-__device__ __forceinline__ double2 cpowf(double2 z, double e) {
-  const double r = pow(hypot(z.x, z.y), e), th = atan2(z.y, z.x) * e;
-  return make_double2(r * cos(th), r * sin(th));
 }
 
 // NormalNormLayer::backward, Complex arm (norm_layer.rs:132-209), one block per
@@ -346,8 +342,9 @@ __global__ __launch_bounds__(256) void k_norm_backward(const double2* __restrict
   const double2 var = cunscale(block_sum2(s, sh), len);
   const double2 sd = csqrt_nc(cadd(var, make_double2(eps, 0.0)));
   const double2 vb = cadd(var, make_double2(1e-8, 0.0));
-  const double2 std_inv = rdivc(1.0, csqrt_nc(vb));
-  const double2 vpm32 = rdivc(1.0, cpowf(vb, 1.5));
+  const double2 vroot = csqrt_nc(vb);
+  const double2 std_inv = rdivc(1.0, vroot);
+  const double2 vpm32 = rdivc(1.0, cmul(vb, vroot));  // powf(1.5) of the principal branch
   double2 P = make_double2(0.0, 0.0), D = P, M = P;
   for (int j = threadIdx.x; j < n; j += 256) {
     const double2 t = csub(xin(j), mu);
