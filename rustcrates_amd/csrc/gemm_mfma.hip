@@ -101,21 +101,27 @@ __device__ __forceinline__ v4d mfma64(double a, double b, v4d c) {
 }
 
 // Tile t of an mt x nt grid: (row, column).  Blocks go to the 8 XCDs in turn
-// and each XCD has its own L2.  In a grid wider than tall the rows run fastest
-// within the blocks of one XCD: a column of tiles, with its slice of the
-// larger operand, belongs to one XCD and is read once (1024 x 32000 x 512,
-// whose 262 MB of weights row order streams 16 times: 2000 -> 1932 us, real A
-// 1191 -> 1116).  Other grids go row by row, where the same for rows measured
-// no gain (16384 x 3072 x 768, real A: 2415 us, 2523 by rows of an XCD).
+// and each XCD has its own L2.  Where one side is short its tiles run fastest
+// within the blocks of one XCD, so that a column (or row) of tiles, with its
+// slice of the larger operand, belongs to one XCD and is read once: 1024 x
+// 32000 x 512, whose 262 MB of weights row order streams 16 times, 2000 ->
+// 1932 us, real A 1191 -> 1116; 4096 x 512 x 2048 498 -> 488.  A tall grid of
+// more columns than an XCD's blocks cover twice goes row by row (16384 x 3072
+// x 768, real A: 2415 us, 2523 by rows of an XCD).
+constexpr int TALL_MAX_COLS = 16;
 __device__ __forceinline__ int2 tile_at(int t, int mt, int nt) {
-  if (nt <= mt) return make_int2(t / nt, t % nt);
-  const int even = nt / 8 * 8;
-  if (t >= even * mt) {
-    const int r = t - even * mt;
-    return make_int2(r % mt, even + r / mt);
+  const bool wide = nt > mt;
+  if (!wide && nt > TALL_MAX_COLS) return make_int2(t / nt, t % nt);
+  const int major = wide ? nt : mt, minor = wide ? mt : nt, even = major / 8 * 8;
+  int a, b;
+  if (t < even * minor) {
+    const int j = t >> 3;
+    a = j / minor * 8 + (t & 7), b = j % minor;
+  } else {
+    const int r = t - even * minor;
+    a = even + r / minor, b = r % minor;
   }
-  const int j = t >> 3;
-  return make_int2(j % mt, j / mt * 8 + (t & 7));
+  return wide ? make_int2(b, a) : make_int2(a, b);
 }
 
 // MODE: the epilogue mode, fixed at compile time so each launch carries only
