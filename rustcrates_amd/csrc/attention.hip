@@ -399,49 +399,62 @@ int attention_decode_split(hipStream_t st, const Attn& a, const double2* q, long
 }
 
 // ===========================================================================
-// Prefill (keys = the S rows of the call, T == S): flash-style, one block per
-// (query tile of 16*NW rows, head, sequence), 32-key tiles up to the tile's
-// causal limit.  Re(q.k) = sum_e (qr kr - qi ki) is a real dot product of
-// length 2*dh: keys are staged in LDS as [kr | -ki], queries held as MFMA A
-// operands [qr | qi], and v_mfma_f64_16x16x4_f64 forms 16x16 score tiles.
-// Scores get the scale and Re(bias_pos[r][c]); keys c > r get -1e12
+// Prefill (keys = the S rows of the call, T == S): flash-style.  A block is NW
+// row waves of 16 query rows times KG key groups; it walks 32-key tiles up to
+// its causal limit, key group g of a row wave taking keys 32 g / KG .. of each
+// tile.  Re(q.k) = sum_e (qr kr - qi ki) is a real dot product of length 2*dh:
+// keys are staged in LDS as [kr | -ki], queries held as MFMA A operands
+// [qr | qi], and v_mfma_f64_16x16x4_f64 forms 16x16 score tiles.  Scores get
+// the scale and Re(bias_pos[r][c]); keys c > r get -1e12
 // (masked_attention_head.rs:189-203).  The softmax runs online (running row
-// max m and sum l, the partial output rescaled by e^(m_old - m_new)); the
-// first tile always holds key 0, so m is a real score from then on and masked
-// keys contribute exactly 0.  P goes through LDS to become the A operand of
-// the P.V MFMAs (values staged in LDS).  out = acc / l; pad rows give 0.
+// max m and sum l, the partial output rescaled by e^(m_old - m_new)); masked keys contribute exactly 0.  P goes through LDS to become the
+// A operand of the P.V MFMAs (values staged in LDS).  Key groups are merged at
+// the end like key chunks; out = acc / l; pad rows give 0.
 // D[i][j] of a 16x16 tile sits at lane j + 16*(i%4), element i/4.
+//
+// Bound by the matrix cores once they are kept busy: the next tile's keys,
+// values and bias rows are requested before this one's products (head dims up
+// to 64), and a wave skips the tiles past its own rows.  Head dims between the
+// built ones run the next wider with zeros.  MI355X, head dim 64, us, against
+// blocks of 128 rows that loaded each tile when it was needed: 48 heads of 1920
+// rows 1822 -> 1573, 768 of 256 765 -> 545, 256 of 128 74 -> 54, 64 of 256 117
+// -> 69, 36 of 173 80 -> 37.  What is left is the softmax: two exponentials per
+// 16 MFMAs in a wave that waits for each tile's scores.
 // ===========================================================================
-template <int DH, int NW>
-__global__ __launch_bounds__(64 * NW) void k_attention_prefill(Attn a) {
+template <int DH, int NW, int KG>
+__global__ __launch_bounds__(64 * NW * KG, DH <= 64 ? 2 : 1) void k_attention_prefill(Attn a) {
   constexpr int KT = 32;          // keys per tile
+  constexpr int JT = KT / 16 / KG;  // 16-key tiles of a wave
   constexpr int KD = 2 * DH;      // real dot length
-  constexpr int KSTR = KD + 1;    // LDS row stride of the key tile (doubles)
-  constexpr int NTH = 64 * NW;
+  constexpr int NTH = 64 * NW * KG;
   constexpr int ET = DH / 16;     // 16-column tiles of the head dim
+  constexpr int PT = KT * DH / NTH;  // key and value elements per thread
+  constexpr bool PRE = DH <= 64;  // the next tile waits in registers
+  constexpr int KSTR = KD + 1, PSTR = KT / KG + 1;  // LDS row strides: a fragment's rows in different banks
   __shared__ double Ks[KT * KSTR];
   __shared__ double2 Vs[KT * DH];
-  __shared__ double Ps[NW][16][KT + 1];
-  const int h = blockIdx.y, b = blockIdx.z;
+  __shared__ double Ps[NW * KG][16 * PSTR];
+  const int h = blockIdx.y, b = blockIdx.z, dh = a.dh;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int rw = wave / KG, kg = wave % KG;
   const int i = lane & 15, kq = lane >> 4;
   const int S = a.S, T = a.T_const;
-  const int q0 = blockIdx.x * 16 * NW;  // block's first query row
-  const int r0 = q0 + 16 * wave;         // wave's first query row
+  const int q0 = (gridDim.x - 1 - blockIdx.x) * 16 * NW;  // block's first query row; the longest blocks start first
+  const int r0 = q0 + 16 * rw;                             // wave's first query row
   const long rowbase = (long)b * S;
-  const double2* Kc = a.kc + ((long)b * a.H + h) * a.ctx * DH;
-  const double2* Vc = a.vc + ((long)b * a.H + h) * a.ctx * DH;
+  const double2* Kc = a.kc + ((long)b * a.H + h) * a.ctx * dh;
+  const double2* Vc = a.vc + ((long)b * a.H + h) * a.ctx * dh;
   const double* bias = a.bias_re + (long)h * a.mc * a.mc;
 
   // A operand of the scores: u[i][k] = k < DH ? qr[k] : qi[k - DH], k = 4s + kq
   double uq[KD / 4];
   {
     const int r = r0 + i;
-    const double2* qrow = a.q + (rowbase + (r < S ? r : 0)) * a.ldq + (long)h * DH;
+    const double2* qrow = a.q + (rowbase + (r < S ? r : 0)) * a.ldq + (long)h * dh;
 #pragma unroll
     for (int s2 = 0; s2 < KD / 4; ++s2) {
-      const int k = 4 * s2 + kq;
-      const double2 qv = r < S ? qrow[k % DH] : make_double2(0.0, 0.0);
+      const int k = 4 * s2 + kq, e = k % DH;
+      const double2 qv = r < S && e < dh ? qrow[e] : make_double2(0.0, 0.0);
       uq[s2] = k < DH ? qv.x : qv.y;
     }
   }
@@ -452,64 +465,147 @@ __global__ __launch_bounds__(64 * NW) void k_attention_prefill(Attn a) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) m[e] = -INFINITY, l[e] = 0.0;
 
+  double2 pk[PRE ? PT : 1], pv[PRE ? PT : 1];
+  auto element = [&](int j, int c0, int& key, int& e) {  // element j of this thread in the tile at c0
+    int idx = tid;
+    asm volatile("" : "+v"(idx));  // its offsets are formed for each tile, not held across the loop
+    idx += NTH * j;
+    key = idx / DH;
+    e = idx - key * DH;
+    return c0 + key < T && e < dh;
+  };
+  auto stage = [&](int key, int e, double2 kv, double2 vv) {
+    Ks[key * KSTR + e] = kv.x;
+    Ks[key * KSTR + DH + e] = -kv.y;
+    Vs[key * DH + e] = vv;
+  };
+  auto fetch = [&](int c0) {
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      int key, e;
+      const bool in = element(j, c0, key, e);
+      pk[j] = in ? Kc[(long)(c0 + key) * dh + e] : make_double2(0.0, 0.0);
+      pv[j] = in ? Vc[(long)(c0 + key) * dh + e] : make_double2(0.0, 0.0);
+    }
+  };
   const int kend = min(T, q0 + 16 * NW);  // keys any row of the block can see
+  if constexpr (PRE) fetch(0);
   for (int c0 = 0; c0 < kend; c0 += KT) {
     __syncthreads();  // the previous tile is consumed
-    for (int idx = tid; idx < KT * DH; idx += NTH) {
-      const int key = idx / DH, e = idx - key * DH, c = c0 + key;
-      const double2 kv = c < T ? Kc[(long)c * DH + e] : make_double2(0.0, 0.0);
-      const double2 vv = c < T ? Vc[(long)c * DH + e] : make_double2(0.0, 0.0);
-      Ks[key * KSTR + e] = kv.x;
-      Ks[key * KSTR + DH + e] = -kv.y;
-      Vs[key * DH + e] = vv;
+    if constexpr (PRE) {
+#pragma unroll
+      for (int j = 0; j < PT; ++j) {
+        int key, e;
+        element(j, c0, key, e);
+        stage(key, e, pk[j], pv[j]);
+      }
+    } else {
+#pragma unroll 4
+      for (int j = 0; j < PT; ++j) {
+        int key, e;
+        const bool in = element(j, c0, key, e);
+        stage(key, e, in ? Kc[(long)(c0 + key) * dh + e] : make_double2(0.0, 0.0),
+              in ? Vc[(long)(c0 + key) * dh + e] : make_double2(0.0, 0.0));
+      }
     }
     __syncthreads();
-    // scores of 16 rows x 32 keys
-    v4d sc[2] = {v4d{0.0, 0.0, 0.0, 0.0}, v4d{0.0, 0.0, 0.0, 0.0}};
+    if constexpr (PRE)
+      if (c0 + KT < kend) fetch(c0 + KT);
+    const int ck = c0 + kg * (KT / KG);  // the wave's first key
+    if (ck > r0 + 15) continue;          // past all its rows (no barrier inside)
+    double bj[4][JT];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int jt = 0; jt < JT; ++jt)
+        bj[e][jt] = bias[(long)min(r0 + 4 * e + kq, S - 1) * a.mc + min(ck + 16 * jt + i, S - 1)];
+    // scores of 16 rows x the wave's keys
+    v4d sc[JT];
+#pragma unroll
+    for (int jt = 0; jt < JT; ++jt) sc[jt] = v4d{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int s2 = 0; s2 < KD / 4; ++s2)
 #pragma unroll
-      for (int jt = 0; jt < 2; ++jt)
-        sc[jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(uq[s2], Ks[(16 * jt + i) * KSTR + 4 * s2 + kq], sc[jt], 0, 0, 0);
+      for (int jt = 0; jt < JT; ++jt)
+        sc[jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(uq[s2], Ks[(kg * (KT / KG) + 16 * jt + i) * KSTR + 4 * s2 + kq],
+                                                      sc[jt], 0, 0, 0);
     // scale, bias, causal mask; online softmax per row
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int r = r0 + 4 * e + kq;
-      double v[2];
+      double v[JT];
       double mt = -INFINITY;
 #pragma unroll
-      for (int jt = 0; jt < 2; ++jt) {
-        const int c = c0 + 16 * jt + i;
-        if (c > r || r >= S) v[jt] = -1e12;
-        else v[jt] = sc[jt][e] * a.scale + bias[(long)r * a.mc + c];
+      for (int jt = 0; jt < JT; ++jt) {
+        const int c = ck + 16 * jt + i;
+        v[jt] = c > r || r >= S ? -1e12 : sc[jt][e] * a.scale + bj[e][jt];
         mt = fmax(mt, v[jt]);
       }
       mt = row16_max(mt);
       const double mn = fmax(m[e], mt);
+      // (skipping the rescale where no max moved spilled 340 registers)
       const double alpha = exp(m[e] - mn);
-      double ls = 0.0;
-#pragma unroll
-      for (int jt = 0; jt < 2; ++jt) {
-        const double p = exp(v[jt] - mn);
-        Ps[wave][4 * e + kq][16 * jt + i] = p;
-        ls += p;
-      }
-      ls = row16_sum(ls);
-      l[e] = l[e] * alpha + ls;
-      m[e] = mn;
 #pragma unroll
       for (int t = 0; t < ET; ++t) o_re[t][e] *= alpha, o_im[t][e] *= alpha;
+      m[e] = mn;
+      double ls = 0.0;
+#pragma unroll
+      for (int jt = 0; jt < JT; ++jt) {
+        const double p = exp(v[jt] - mn);
+        Ps[wave][(4 * e + kq) * PSTR + 16 * jt + i] = p;
+        ls += p;
+      }
+      l[e] = l[e] * alpha + row16_sum(ls);
     }
-    __syncthreads();  // P of every wave written
+    __builtin_amdgcn_wave_barrier();  // P is the wave's own: LDS keeps a wave's accesses in order
     // out += P . V: A = P[row i][key 4s + kq], B = V[key 4s + kq][16t + i]
 #pragma unroll
-    for (int s2 = 0; s2 < KT / 4; ++s2) {
-      const double pa = Ps[wave][i][4 * s2 + kq];
+    for (int s2 = 0; s2 < KT / KG / 4; ++s2) {
+      const double pa = Ps[wave][i * PSTR + 4 * s2 + kq];
 #pragma unroll
       for (int t = 0; t < ET; ++t) {
-        const double2 vb = Vs[(4 * s2 + kq) * DH + 16 * t + i];
+        const double2 vb = Vs[(kg * (KT / KG) + 4 * s2 + kq) * DH + 16 * t + i];
         o_re[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa, vb.x, o_re[t], 0, 0, 0);
         o_im[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa, vb.y, o_im[t], 0, 0, 0);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if constexpr (KG > 1) {
+    // key group 0 of each row wave takes the others' (max, sum, output) in
+    // order, rescaled to the common max; the tiles' LDS is free by then.  Group
+    // 0 has seen key 0, so its max is a score; a group whose rows saw only
+    // masked keys (max -1e12, or none) weighs e^-inf = 0.
+    __syncthreads();
+    constexpr int HALF = NW * 64 * 4 * ET;  // doubles of one part
+    double* mo = (double*)Vs;               // [NW][4 ET][64] real parts
+    double* mi = Ks;                        // imaginary parts
+    double* ml = &Ps[0][0];                 // [NW][4 max, 4 sum][64]
+    static_assert(KG == 2 && sizeof(double) * HALF <= sizeof(Vs) && sizeof(double) * HALF <= sizeof(Ks) &&
+                      sizeof(double) * NW * 64 * 8 <= sizeof(Ps), "merge buffers");
+    if (kg == 1) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+#pragma unroll
+        for (int t = 0; t < ET; ++t) {
+          mo[((rw * ET + t) * 4 + e) * 64 + lane] = o_re[t][e];
+          mi[((rw * ET + t) * 4 + e) * 64 + lane] = o_im[t][e];
+        }
+        ml[(rw * 8 + e) * 64 + lane] = m[e];
+        ml[(rw * 8 + 4 + e) * 64 + lane] = l[e];
+      }
+    }
+    __syncthreads();
+    if (kg == 1) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const double m1 = ml[(rw * 8 + e) * 64 + lane], l1 = ml[(rw * 8 + 4 + e) * 64 + lane];
+      const double mn = fmax(m[e], m1), w0 = exp(m[e] - mn), w1 = exp(m1 - mn);
+      l[e] = l[e] * w0 + l1 * w1;
+#pragma unroll
+      for (int t = 0; t < ET; ++t) {
+        o_re[t][e] = o_re[t][e] * w0 + mo[((rw * ET + t) * 4 + e) * 64 + lane] * w1;
+        o_im[t][e] = o_im[t][e] * w0 + mi[((rw * ET + t) * 4 + e) * 64 + lane] * w1;
       }
     }
   }
@@ -519,25 +615,33 @@ __global__ __launch_bounds__(64 * NW) void k_attention_prefill(Attn a) {
     if (r >= S) continue;
     const long row = rowbase + r;
     const bool pad = a.row_mask && a.row_mask[row] == 0;
-    double2* out = a.out + row * a.ldo + (long)h * DH;
+    double2* out = a.out + row * a.ldo + (long)h * dh;
 #pragma unroll
     for (int t = 0; t < ET; ++t)
-      out[16 * t + i] = pad ? make_double2(0.0, 0.0) : make_double2(o_re[t][e] / l[e], o_im[t][e] / l[e]);
+      if (16 * t + i < dh)
+        out[16 * t + i] = pad ? make_double2(0.0, 0.0) : make_double2(o_re[t][e] / l[e], o_im[t][e] / l[e]);
   }
 }
 
+// 128 rows per block share each tile where that gives two blocks per CU; short
+// of it, 64 or 32 rows with two key groups (us with 32 / 64 rows: 64 heads of
+// 256 rows 79 / 69, 64 of 128 35 / 39, 36 of 173 37 / 49)
 bool attention_prefill(hipStream_t st, const Attn& a) {
-  if (a.kv_len || a.T_const != a.S || a.S <= 0) return false;
-  const auto launch = [&](auto kern, int nw) {
-    MITOK_LAUNCH(kern, dim3(cdiv_i(a.S, 16 * nw), a.H, a.B), dim3(64 * nw), 0, st, a);
+  if (a.kv_len || a.T_const != a.S || a.S <= 0 || a.dh > 128) return false;
+  const auto launch = [&](auto kern, int nw, int kg) {
+    MITOK_LAUNCH(kern, dim3(cdiv_i(a.S, 16 * nw), a.H, a.B), dim3(64 * nw * kg), 0, st, a);
   };
-  switch (a.dh) {
-    case 16: launch(k_attention_prefill<16, 8>, 8); return true;
-    case 32: launch(k_attention_prefill<32, 8>, 8); return true;
-    case 64: launch(k_attention_prefill<64, 8>, 8); return true;
-    case 128: launch(k_attention_prefill<128, 4>, 4); return true;
-    default: return false;
-  }
+  const auto sized = [&](auto rows32, auto rows64, auto rows128) {
+    const long blocks64 = (long)cdiv_i(a.S, 64) * a.H * a.B;
+    if (blocks64 < 256) launch(rows32, 2, 2);
+    else if (blocks64 < 512) launch(rows64, 4, 2);
+    else launch(rows128, 8, 1);
+  };
+  if (a.dh <= 16) sized(k_attention_prefill<16, 2, 2>, k_attention_prefill<16, 4, 2>, k_attention_prefill<16, 8, 1>);
+  else if (a.dh <= 32) sized(k_attention_prefill<32, 2, 2>, k_attention_prefill<32, 4, 2>, k_attention_prefill<32, 8, 1>);
+  else if (a.dh <= 64) sized(k_attention_prefill<64, 2, 2>, k_attention_prefill<64, 4, 2>, k_attention_prefill<64, 8, 1>);
+  else launch(k_attention_prefill<128, 4, 1>, 4, 1);
+  return true;
 }
 
 }  // namespace mitok

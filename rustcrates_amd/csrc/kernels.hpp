@@ -150,8 +150,8 @@ struct Attn {
 };
 // One query row per block (the general reference case, any T).
 void attention_rows(hipStream_t st, const Attn& a);
-// Prefill (T == S, no KV length): tiled MFMA kernel for head dims 16, 32, 64,
-// 128; returns false (nothing launched) for other shapes.
+// Prefill (T == S, no KV length): tiled MFMA kernel for head dims up to 128;
+// returns false (nothing launched) for other shapes.
 bool attention_prefill(hipStream_t st, const Attn& a);
 // Decode (S == 1): key chunks in parallel; the chunk partials (AttnSplit) are
 // combined by a RowOps prologue (rowops_apply or a GEMV).  q is the sum of
