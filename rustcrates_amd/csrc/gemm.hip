@@ -662,9 +662,33 @@ __global__ __launch_bounds__(256) void k_zgemm_skinny_rows(const double2* __rest
 // four waves per SIMD).  The 16 waves' tiles are summed through LDS in wave
 // order, so results repeat bit for bit.
 // ===========================================================================
+// REAL: the rows' imaginary parts are zero (a Norm's output, as QKV and FFN
+// Dense read): their real parts alone are loaded and two MFMAs a step form the
+// product; where the weights hold an infinity or NaN the sums 0 * that would
+// have entered become NaN (as in gemm_mfma.hip).  64 rows, FFN Dense 768 x
+// 3072: 38 -> 29 us; 32 rows at width 512 stay at 9.9, bound by latency.
 constexpr int ROWS16_WAVES = 16;
 constexpr size_t ROWS16_LDS = (size_t)ROWS16_WAVES * 16 * 16 * sizeof(double2);  // 64 KB
 
+// what a real-row product makes of its weights' non-finite parts: top_re,
+// top_im the largest high words (sign off) a lane loaded of its column
+__device__ __forceinline__ void poison_columns(int top_re, int top_im, v4d& cr, v4d& ci) {
+  const unsigned long long re = __ballot(top_re >= 0x7ff00000), im = __ballot(top_im >= 0x7ff00000);
+  if ((re | im) == 0) return;
+  const int i = threadIdx.x & 15;
+  if ((im >> i | im >> (i + 16) | im >> (i + 32) | im >> (i + 48)) & 1) cr = v4d{NAN, NAN, NAN, NAN};
+  if ((re >> i | re >> (i + 16) | re >> (i + 32) | re >> (i + 48)) & 1) ci = v4d{NAN, NAN, NAN, NAN};
+}
+__device__ __forceinline__ void top_words(double2 v, int& re, int& im) {
+  re = max(re, __double2hiint(v.x) & 0x7fffffff);
+  im = max(im, __double2hiint(v.y) & 0x7fffffff);
+}
+__device__ __forceinline__ double part_re(double v) { return v; }
+__device__ __forceinline__ double part_re(double2 v) { return v.x; }
+__device__ __forceinline__ double part_im(double) { return 0.0; }
+__device__ __forceinline__ double part_im(double2 v) { return v.y; }
+
+template <bool REAL>
 __global__ __launch_bounds__(1024) void k_zgemm_rows16(const double2* __restrict__ X, long ldx, int M,
                                                      const double2* __restrict__ W, long ldw, int N, int K, int nkw,
                                                      Epi ep) {
@@ -674,13 +698,17 @@ __global__ __launch_bounds__(1024) void k_zgemm_rows16(const double2* __restrict
   const int i = lane & 15, kq = lane >> 4;
   const int n = blockIdx.x * 16 + i, m = blockIdx.y * 16 + i;
   const int ka = (blockIdx.z * NW + wave) * 4 * nkw, kz = min(K, ka + 4 * nkw);
-  double2 a[2][U], b[2][U];
+  typedef typename std::conditional<REAL, double, double2>::type TA;
+  TA a[2][U];
+  double2 b[2][U];
+  int top_re = 0, top_im = 0;
   auto load = [&](int s, int k) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int kk = k + 4 * u + kq;
       b[s][u] = (kk < kz && n < N) ? W[(long)kk * ldw + n] : make_double2(0.0, 0.0);
-      a[s][u] = (kk < kz && m < M) ? X[(long)m * ldx + kk] : make_double2(0.0, 0.0);
+      if constexpr (REAL) a[s][u] = (kk < kz && m < M) ? X[(long)m * ldx + kk].x : 0.0;
+      else a[s][u] = (kk < kz && m < M) ? X[(long)m * ldx + kk] : make_double2(0.0, 0.0);
     }
   };
   v4d cr = {0.0, 0.0, 0.0, 0.0}, ci = {0.0, 0.0, 0.0, 0.0};
@@ -689,10 +717,14 @@ __global__ __launch_bounds__(1024) void k_zgemm_rows16(const double2* __restrict
   auto mma = [&](int s) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][u].x, b[s][u].x, cr, 0, 0, 0);
-      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][u].x, b[s][u].y, ci, 0, 0, 0);
-      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[s][u].y, b[s][u].y, cr, 0, 0, 0);
-      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][u].y, b[s][u].x, ci, 0, 0, 0);
+      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(part_re(a[s][u]), b[s][u].x, cr, 0, 0, 0);
+      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(part_re(a[s][u]), b[s][u].y, ci, 0, 0, 0);
+      if constexpr (REAL) {
+        top_words(b[s][u], top_re, top_im);
+      } else {
+        cr = __builtin_amdgcn_mfma_f64_16x16x4f64(-part_im(a[s][u]), b[s][u].y, cr, 0, 0, 0);
+        ci = __builtin_amdgcn_mfma_f64_16x16x4f64(part_im(a[s][u]), b[s][u].x, ci, 0, 0, 0);
+      }
     }
   };
   constexpr int KS = 4 * U;  // k per batch; unrolled by two so buffer indices are constants
@@ -705,6 +737,7 @@ __global__ __launch_bounds__(1024) void k_zgemm_rows16(const double2* __restrict
     mma(1);
     if (k + 3 * KS < kz) load(1, k + 3 * KS);
   }
+  if constexpr (REAL) poison_columns(top_re, top_im, cr, ci);
 #pragma unroll
   for (int e = 0; e < 4; ++e) red16[(wave * 16 + 4 * e + kq) * LD + i] = make_double2(cr[e], ci[e]);
   __syncthreads();
@@ -733,7 +766,7 @@ __global__ __launch_bounds__(1024) void k_zgemm_rows16(const double2* __restrict
 // in ascending order) is the same as there, so the results are identical.
 __device__ const double2 rows16s_zero = {0.0, 0.0};  // what an out-of-range operand lane reads
 
-template <int NB>  // batches of 2 k-steps: 4 (32 of K per wave, 512 per block) or 6 (48, 768)
+template <int NB, bool REAL>  // batches of 2 k-steps: 4 (32 of K per wave, 512 per block) or 6 (48, 768)
 __global__ __launch_bounds__(1024) void k_zgemm_rows16s(const double2* __restrict__ X, long ldx, int M,
                                                       const double2* __restrict__ W, long ldw, int N, int K, Epi ep) {
   constexpr int U = 2, NW = ROWS16_WAVES, LD = 16;
@@ -744,7 +777,9 @@ __global__ __launch_bounds__(1024) void k_zgemm_rows16s(const double2* __restric
   const int ka = (blockIdx.z * NW + wave) * 8 * NB;
   const long nc = min(n, N - 1), mc = min(m, M - 1);
   const bool nok = n < N, mok = m < M;
-  double2 a[NB][U], b[NB][U];
+  typedef typename std::conditional<REAL, double, double2>::type TA;
+  TA a[NB][U];
+  double2 b[NB][U];
 #pragma unroll
   for (int s = 0; s < NB; ++s)
 #pragma unroll
@@ -755,18 +790,26 @@ __global__ __launch_bounds__(1024) void k_zgemm_rows16s(const double2* __restric
       const long kc = min(kk, K - 1);
       const bool ok = kk < K;
       b[s][u] = ld_glb((ok && nok) ? W + kc * ldw + nc : &rows16s_zero);
-      a[s][u] = ld_glb((ok && mok) ? X + mc * ldx + kc : &rows16s_zero);
+      const double2* pa = (ok && mok) ? X + mc * ldx + kc : &rows16s_zero;
+      if constexpr (REAL) a[s][u] = ld_glb(&pa->x);
+      else a[s][u] = ld_glb(pa);
     }
   v4d cr = {0.0, 0.0, 0.0, 0.0}, ci = {0.0, 0.0, 0.0, 0.0};
+  int top_re = 0, top_im = 0;
 #pragma unroll
   for (int s = 0; s < NB; ++s)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][u].x, b[s][u].x, cr, 0, 0, 0);
-      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][u].x, b[s][u].y, ci, 0, 0, 0);
-      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[s][u].y, b[s][u].y, cr, 0, 0, 0);
-      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][u].y, b[s][u].x, ci, 0, 0, 0);
+      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(part_re(a[s][u]), b[s][u].x, cr, 0, 0, 0);
+      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(part_re(a[s][u]), b[s][u].y, ci, 0, 0, 0);
+      if constexpr (REAL) {
+        top_words(b[s][u], top_re, top_im);
+      } else {
+        cr = __builtin_amdgcn_mfma_f64_16x16x4f64(-part_im(a[s][u]), b[s][u].y, cr, 0, 0, 0);
+        ci = __builtin_amdgcn_mfma_f64_16x16x4f64(part_im(a[s][u]), b[s][u].x, ci, 0, 0, 0);
+      }
     }
+  if constexpr (REAL) poison_columns(top_re, top_im, cr, ci);
 #pragma unroll
   for (int e = 0; e < 4; ++e) red16[(wave * 16 + 4 * e + kq) * LD + i] = make_double2(cr[e], ci[e]);
   __syncthreads();
@@ -1119,7 +1162,11 @@ static SkinnyPlan plan_skinny(int M, int N, int K, bool part, bool argmax) {
     r.w16 = 1;
     r.ct = 1;
     r.ncb = cdiv_i(N, 16);
-    r.nkw = 8;
+    // 768 of K per block where that divides K and the grid still fills the
+    // chip: K 768 in 512s leaves half the second block's waves idle and a
+    // partial more for the consumer (64 rows at width 768, the layer products
+    // of a decode step together, with the real rows below: 106 -> 94 us)
+    r.nkw = K % 768 == 0 && (long)r.ncb * r.rt * (K / 768) >= 256 && K / 768 <= SKINNY_MAX_SPLIT ? 12 : 8;
     int P = cdiv_i(K, 64 * r.nkw);
     if (!part) {
       r.nkw = cdiv_i(K, 64);
@@ -1265,9 +1312,14 @@ static void launch_skinny(hipStream_t st, const SkinnyPlan& p, const RowOps& ro,
   if (p.rows) {  // EPI_PART, or one K range per block (no argmax: not a vocab-wide output)
     const dim3 g3(p.ncb, p.rt, p.P);
     if (p.w16) {
-      if (p.nkw == 8) MITOK_LAUNCH(k_zgemm_rows16s<4>, g3, dim3(64 * ROWS16_WAVES), ROWS16_LDS, st, ro.x, ro.ldx, M, W, ldw, N, K, ep);
-      else if (p.nkw == 12) MITOK_LAUNCH(k_zgemm_rows16s<6>, g3, dim3(64 * ROWS16_WAVES), ROWS16_LDS, st, ro.x, ro.ldx, M, W, ldw, N, K, ep);
-      else MITOK_LAUNCH(k_zgemm_rows16, g3, dim3(64 * ROWS16_WAVES), ROWS16_LDS, st, ro.x, ro.ldx, M, W, ldw, N, K, p.nkw, ep);
+      const dim3 b16(64 * ROWS16_WAVES);
+      const auto go = [&](auto kern8, auto kern12, auto kern) {
+        if (p.nkw == 8) MITOK_LAUNCH(kern8, g3, b16, ROWS16_LDS, st, ro.x, ro.ldx, M, W, ldw, N, K, ep);
+        else if (p.nkw == 12) MITOK_LAUNCH(kern12, g3, b16, ROWS16_LDS, st, ro.x, ro.ldx, M, W, ldw, N, K, ep);
+        else MITOK_LAUNCH(kern, g3, b16, ROWS16_LDS, st, ro.x, ro.ldx, M, W, ldw, N, K, p.nkw, ep);
+      };
+      if (ro.real) go(k_zgemm_rows16s<4, true>, k_zgemm_rows16s<6, true>, k_zgemm_rows16<true>);
+      else go(k_zgemm_rows16s<4, false>, k_zgemm_rows16s<6, false>, k_zgemm_rows16<false>);
       return;
     }
     if (p.ct == 2) MITOK_LAUNCH(k_zgemm_skinny_rows<2>, g3, blk, 0, st, ro.x, ro.ldx, M, W, ldw, N, K, p.nkw, ep);

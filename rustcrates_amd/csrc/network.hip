@@ -1066,7 +1066,7 @@ static int enqueue_decode_fused(Net* n, const Spec& sp) {
     double2* out = mats[mat_next];
     mat_next ^= 1;
     rowops_apply(st, B, width, pro, out, width);
-    RowOps r = rows_of(out, width);
+    RowOps r = rows_of(out, width, pro.ln || pro.resid || (pro.real && pro.plain()));
     r.err = err;
     pro = r;
   };
@@ -1122,9 +1122,10 @@ static int enqueue_decode_fused(Net* n, const Spec& sp) {
         // decode per step 763 -> 708 us at config 3 with 8 sequences, 496 ->
         // 489 with 4, 1943 -> 1911 at config 5 with 4
         if (mat || B >= FUSED_PLAIN_MIN_B) {
+          const bool real = pro.ln || pro.resid || (pro.real && pro.plain());  // Re(..) + 0i either way
           if (!pro.plain()) rowops_apply(st, B, d, pro, x1, d);
           else x1 = const_cast<double2*>(pro.x);  // a materialised row buffer (ld d), not reused before the combine
-          pro = rows_of(x1, d);
+          pro = rows_of(x1, d, real);
           pro.err = err;
         } else {
           pro.save = x1;

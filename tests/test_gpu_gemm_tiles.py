@@ -20,6 +20,8 @@ EPS = np.finfo(np.float64).eps
 # of every tile (fewer than 256 tiles), whole tiles and split ones (over 256)
 SHAPES = [(65, 8, 64), (65, 9, 63), (127, 7, 65), (64 * 3, 100, 130), (70, 1024, 64), (130, 777, 96),
           (519, 264, 2304), (257 * 64, 16, 64)]
+# at most 64 rows: the row-tile products, straight-line (512 and 768 of K) and looped
+SKINNY = [(9, 512, 64), (33, 768, 33), (64, 512, 1000), (17, 300, 48), (64, 1000, 20), (20, 257, 17)]
 
 
 def linear_net(d, n, seed, w=None):
@@ -41,7 +43,7 @@ def close(got, a, w, b):
         assert np.all(over <= 0), float(over.max())
 
 
-@pytest.mark.parametrize("rows,k,n", SHAPES)
+@pytest.mark.parametrize("rows,k,n", SHAPES + SKINNY)
 def test_tiled_product_on_complex_and_real_rows(rows, k, n):
     net, w, b = linear_net(k, n, rows + k + n)
     r = np.random.default_rng(rows)
@@ -55,9 +57,10 @@ def test_tiled_product_on_complex_and_real_rows(rows, k, n):
     close(z, h, w, b)
 
 
-def test_real_rows_meet_infinities_and_nan_as_complex_ones_do():
+@pytest.mark.parametrize("rows,k", [(70, 40), (20, 512), (20, 300)])
+def test_real_rows_meet_infinities_and_nan_as_complex_ones_do(rows, k):
     """A product with zero imaginary parts left out must still give NaN where 0 * (infinity or NaN) would."""
-    k, n, rows = 40, 80, 70
+    n = 80
     r = np.random.default_rng(3)
     w = r.standard_normal((k, n)) + 1j * r.standard_normal((k, n))
     w[3, 2] = complex(np.inf, 1.0)
