@@ -70,16 +70,25 @@ def kernel_class(net, prompt, lens, n_new, cls, reps=2):
     return r
 
 
+def real_rows_share(c):
+    """Flops a block's products need, as a share of 8 per multiply-add (which
+    the library's layer_gemm and prefill_gemm classes count): Q/K/V and FFN
+    Dense read real rows."""
+    qkv, ffn = 3.0 * c.d * c.d, 1.0 * c.d * c.ffn
+    return (0.5 * (qkv + ffn) + ffn) / (qkv + 2 * ffn)
+
+
 def prefill_flops(w, lens):
-    """Algorithmic flops of the prompt pass: 8 per complex multiply-add of the
-    Q/K/V and FFN products over every prompt row, the causal half of Re(q.k)
-    (8 per key) and of P.V (4, real x complex), and the vocab product of each
-    sequence's last row only."""
+    """Algorithmic flops of the prompt pass: the Q/K/V and FFN Dense products
+    of every prompt row at 4 per multiply-add (a Norm leaves real rows), FFN
+    Linear at 8, the causal half of Re(q.k) (8 per key) and of P.V (4, real x
+    complex), and the vocab product's real part (4) of each sequence's last
+    row only."""
     c = w.model
     rows = float(sum(lens))
-    proj = 8.0 * c.layers * rows * (3 * c.d * c.d + 2 * c.d * c.ffn)
+    proj = real_rows_share(c) * 8.0 * c.layers * rows * (3 * c.d * c.d + 2 * c.d * c.ffn)
     attn = c.layers * sum(12.0 * c.d * s * (s + 1) / 2 for s in lens)
-    vocab = 8.0 * len(lens) * c.d * c.vocab
+    vocab = 4.0 * len(lens) * c.d * c.vocab
     return proj + attn + vocab
 
 
@@ -220,6 +229,8 @@ def run(args, w, net):
         for name, cls in (("vocab", ra.TIME_VOCAB), ("layer_gemm", ra.TIME_LAYER_GEMM),
                           ("attention", ra.TIME_ATTENTION), ("prefill_gemm", ra.TIME_PREFILL_GEMM)):
             classes[name] = kernel_class(net, prompt, lens, n_new, cls)
+            if name in ("layer_gemm", "prefill_gemm"):
+                classes[name]["alg_flops"] *= real_rows_share(cfg)
         # the dominant class of the decode step (the prompt pass has its own
         # entry below); a class is MFMA-bound when its arithmetic intensity
         # exceeds the ridge point, else HBM-bound
@@ -309,8 +320,9 @@ def head_train_step(cfg, B=8, S=128, T=64, reps=5):
     """The output head's training step (mitok_backward_head: Softmax
     cross-entropy gradient, vocab Linear backward, then its AdamW update) at
     config 3's head shapes, after one TRAINING-mode predict of B x S rows.
-    Algorithmic flops: the two products dW = conj(X)^T G and dX = G conj(W)^T,
-    8 * d * V * rows each."""
+    Algorithmic flops: the two products dW = conj(X)^T G and dX = G conj(W)^T
+    over the rows with a target (G is real, and zero in the others), 4 * d * V
+    * rows each."""
     with ra.Network(0) as h:
         h.add_embedding(cfg.vocab, cfg.d)
         h.add_linear(cfg.d, cfg.vocab)
@@ -326,7 +338,7 @@ def head_train_step(cfg, B=8, S=128, T=64, reps=5):
         for t in range(reps):
             h.backward_head(targets, update=True, learning_rate=1e-3, time_step=3 + t, want_grad_input=False)
         ms = (time.perf_counter() - t0) / reps * 1e3
-    flops = 2 * 8.0 * cfg.d * cfg.vocab * B * S
+    flops = 2 * 4.0 * cfg.d * cfg.vocab * B * T
     return {"config": f"vocab Linear {cfg.d} x {cfg.vocab}, {B} x {S} rows, {T} targets per sequence, AdamW update",
             "ms_per_step": round(ms, 3), "alg_gflop": round(flops / 1e9, 2),
             "tflops": round(flops / (ms / 1e3) / 1e12, 3),
@@ -339,10 +351,11 @@ def train_step(cfg, B=8, S=128, T=64, reps=3):
     cross_entropy_loss_batch on its softmax output, both on the device (only
     the loss crosses PCIe, mitok_cross_entropy_loss), then backward over every
     layer with every update (mitok_backward).  Algorithmic flops of the
-    backward's products (8 M N K each): per attention layer the Q/K/V
-    recompute, their weight and input gradients (3 x 24 rows d^2); per
-    FeedForward the Dense recompute twice and four gradient products
-    (6 x 8 rows d F); the vocab Linear's two (16 rows d V)."""
+    backward's products, 8 per multiply-add and 4 where an operand is real:
+    per attention layer the Q/K/V weight and input gradients (3 x 12 rows
+    d^2); per FeedForward four gradient products (20 rows d F, 8 more in the
+    top one, whose gradient is complex); the vocab Linear's two over the rows
+    with a target (4 d V each)."""
     rows = B * S
     with ra.Network(0) as net:
         configs.build_network(net, cfg, mode=ra.TRAINING)
@@ -366,7 +379,7 @@ def train_step(cfg, B=8, S=128, T=64, reps=3):
             bwd += time.perf_counter() - t1
     fwd_ms, bwd_ms = fwd / reps * 1e3, bwd / reps * 1e3
     d, F, V = cfg.d, cfg.ffn, cfg.vocab
-    flops = cfg.layers * (3 * 24.0 * rows * d * d + 6 * 8.0 * rows * d * F) + 16.0 * rows * d * V
+    flops = cfg.layers * (3 * 12.0 * rows * d * d + 20.0 * rows * d * F) + 8.0 * rows * d * F + 8.0 * B * T * d * V
     return {"config": f"{cfg.name}, {B} x {S} rows, {T} targets per sequence, backward over all {nl - 1} "
                       "layers below the Softmax with every update",
             "forward_ms": round(fwd_ms, 3), "backward_ms": round(bwd_ms, 3),
