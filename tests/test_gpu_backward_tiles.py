@@ -1,7 +1,7 @@
 """Backward's tiled products where their tiles and row packing change: the
 head's packed target rows (gemm_mfma.hip's transposed operands, real
 gradients), and the attention heads' products at the widths where the row
-kernel takes another number of values per lane, against the CPU checker.
+kernel takes another number of values per lane, against the CPU oracle.
 
 Bar: within 1e-11 of the largest element, as in test_gpu_train.py (the
 products sum in another order; the weights are scaled so that every gradient
