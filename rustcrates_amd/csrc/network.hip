@@ -73,6 +73,7 @@ struct DevBuf {
     size_t want = std::max<size_t>(n, 256);
     hipError_t e = hipMalloc(&p, want);
     if (e != hipSuccess) {
+      (void)hipGetLastError();  // kept until it is read: a later call would take it for its own
       p = nullptr;
       return fail(ERR_NOMEM, "hipMalloc(%zu bytes): %s", want, hipGetErrorString(e));
     }
