@@ -283,8 +283,9 @@ struct Spec {
   bool forward_only = true;
   bool last_row = false;
   uint32_t first = 0, last = 0;      // layer range
-  const double2* in = nullptr;       // hidden-state input when first > 0
-  const uint32_t* ids = nullptr;     // [B*S] padded ids (first == 0)
+  bool hidden = false;               // a hidden-state range: rows in, rows out, every Linear an ordinary one
+  const double2* in = nullptr;       // its input
+  const uint32_t* ids = nullptr;     // else: [B*S] padded ids
   const uint32_t* mask = nullptr;    // [B*S]
   const uint32_t* lens = nullptr;    // [B]
   const int* pos = nullptr;          // [B*S] RoPE positions, or null -> kv_len (S == 1)
@@ -566,8 +567,8 @@ static bool is_vocab_linear(const Net* n, uint32_t li) {
   return n->layers[li]->kind == K_LINEAR && li + 2 == n->layers.size() && n->layers.back()->kind == K_SOFTMAX;
 }
 
-// a stateless pass from the Embedding on is what backward may differentiate
-static bool keeps(const Spec& sp) { return sp.mode == MODE_STATELESS && sp.first == 0; }
+// a stateless pass of the whole stack is what backward may differentiate
+static bool keeps(const Spec& sp) { return sp.mode == MODE_STATELESS && !sp.hidden; }
 
 // Gives up the saved forward products: backward then forms them again.
 static void drop_saved(Net* n) {
@@ -628,7 +629,7 @@ static int prepare(Net* n, const Spec& sp) {
       product(M, F->d_out, F->hidden);
     }
     if (L->kind == K_LINEAR) {
-      const bool vocab = is_vocab_linear(n, li) && sp.first == 0;
+      const bool vocab = is_vocab_linear(n, li) && !sp.hidden;
       const int Mv = (vocab && sp.last_row) ? sp.B : M;
       product(Mv, L->d_out, L->d_in);
       if (vocab && !sp.forward_only) {
@@ -906,7 +907,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
       }
       case K_LINEAR: {
         auto* Ln = (LinearLayer*)L;
-        const bool vocab = is_vocab_linear(n, li) && sp.first == 0;
+        const bool vocab = is_vocab_linear(n, li) && !sp.hidden;
         if (!vocab) {
           Epi e;
           e.mode = EPI_STORE;
@@ -2492,6 +2493,7 @@ static int forward_layers_impl(Net* n, uint32_t first, uint32_t last, const doub
     TRY(check_device_range(n, out, (size_t)B * so * dout * sizeof(double2), "out"));
   }
   Spec sp;
+  sp.hidden = true;
   sp.first = first;
   sp.last = last;
   std::vector<uint32_t> mask_h;

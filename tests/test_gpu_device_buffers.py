@@ -89,3 +89,35 @@ def test_device_entry_points_refuse_host_and_short_buffers():
         assert g.forward_layers_device(1, 3, din, B, S, dout) == S
         assert np.array_equal(dout.download((B, S, d), np.complex128), g.forward_layers(1, 3, x))
     g.close()
+
+
+@pytest.mark.parametrize("rows", [5, 40, 70])
+@pytest.mark.parametrize("forward_only", [False, True])
+def test_a_range_ends_in_the_vocabulary_linear(rows, forward_only):
+    """A layer range takes rows and gives rows: the Linear before a Softmax is
+    an ordinary product there, from the first layer of a stack too, and leaves
+    nothing to differentiate.  Bound as in test_gpu_gemm_tiles.py: (K + 4) eps
+    of the sums of magnitudes."""
+    d, V = 24, 90
+    r = np.random.default_rng(rows)
+    w = r.standard_normal((d, V)) + 1j * r.standard_normal((d, V))
+    b = r.standard_normal(V) + 1j * r.standard_normal(V)
+    x = r.standard_normal((1, rows, d)) + 1j * r.standard_normal((1, rows, d))
+    with ra.Network(0) as g:
+        g.add_norm(d, 1e-5)
+        g.add_linear(d, V, w, b)
+        g.add_softmax(ra.TRAINING)
+        h = g.forward_layers(0, 1, x, forward_only=forward_only)
+        g.reset()
+        host = g.forward_layers(0, 2, x, forward_only=forward_only, d_out=V)
+        with ra.DeviceBuffer(x.nbytes) as din, ra.DeviceBuffer(host.nbytes) as dout:
+            din.upload(x)
+            g.reset()
+            g.forward_layers_device(0, 2, din.ptr, dout.ptr, 1, rows, forward_only=forward_only)
+            dev = dout.download(host.shape, np.complex128)
+        with pytest.raises(ra.MitokError, match="no stateless"):
+            g.backward_head(np.full((1, 2), 3, np.uint32), update=False)
+    assert np.array_equal(dev, host)
+    want = h[0] @ w + b
+    bound = (d + 4) * np.finfo(np.float64).eps * (np.abs(h[0]) @ np.abs(w) + np.abs(b))
+    assert np.all(np.abs(host[0].real - want.real) <= bound) and np.all(np.abs(host[0].imag - want.imag) <= bound)
