@@ -113,7 +113,7 @@ def test_a_range_ends_in_the_vocabulary_linear(rows, forward_only):
         with ra.DeviceBuffer(x.nbytes) as din, ra.DeviceBuffer(host.nbytes) as dout:
             din.upload(x)
             g.reset()
-            g.forward_layers_device(0, 2, din.ptr, dout.ptr, 1, rows, forward_only=forward_only)
+            g.forward_layers_device(0, 2, din, 1, rows, dout, forward_only=forward_only)
             dev = dout.download(host.shape, np.complex128)
         with pytest.raises(ra.MitokError, match="no stateless"):
             g.backward_head(np.full((1, 2), 3, np.uint32), update=False)
