@@ -297,7 +297,8 @@ struct Spec {
   bool compress = false;             // apply the wavelet stages begin_call planned for this call
   double* hist_re = nullptr;         // Re-logits history [step][B][V] at hist_cnt[0] (token loop)
   const int* hist_cnt = nullptr;
-  int S_out = 0;                     // sizing: rows per sequence after a compression (0: S)
+  int S_first = 0, T = 0;            // sizing: rows per sequence before the call's compressions (0: none
+                                     // follow; S is the most they reach) and its target rows
   int ctx_bound = 0;                 // keys a decode step of this call can reach (0: the layers' context)
 };
 
@@ -591,6 +592,12 @@ static int reserve_saved(Net* n, const Spec& sp, size_t rows) {
   return OK;
 }
 
+// rows per sequence that a wavelet layer of a prompt or stateless pass leaves
+// of S: it compresses all but the last T, the target rows
+static int compressed_rows(const WaveletLayer* W, int S, int T) {
+  return T ? wavelet_rows(S - T, W->L) + T : wavelet_rows(S, W->L);
+}
+
 static int prepare(Net* n, const Spec& sp) {
   n->head_valid = false;  // the workspaces that held the last stateless pass's head input are reused
   const Dims dm = net_dims(n);
@@ -615,13 +622,12 @@ static int prepare(Net* n, const Spec& sp) {
     }
   }
   size_t ws = 0;
-  const auto product = [&](int m, int N, int K) {  // split workspace of a product, before or after a compression
-    ws = std::max(ws, gemm_ws_bytes(m, N, K));
-    if (sp.S_out && m == (int)rows) ws = std::max(ws, gemm_ws_bytes(sp.B * sp.S_out, N, K));
-  };
+  const auto product = [&](int m, int N, int K) { ws = std::max(ws, gemm_ws_bytes(m, N, K)); };
+  // each product at the rows it runs on: more rows may need less workspace (a whole round of tiles is not split)
+  int M = sp.B * (sp.S_first ? sp.S_first : sp.S);
   for (uint32_t li = sp.first; li < sp.last; ++li) {
     Layer* L = n->layers[li].get();
-    const int M = (int)rows;
+    if (L->kind == K_WAVELET && sp.S_first) M = sp.B * compressed_rows((const WaveletLayer*)L, M / sp.B, sp.T);
     if (L->kind == K_SELF_ATTENTION) product(M, 3 * L->d_in, L->d_in);
     if (L->kind == K_FEED_FORWARD) {
       auto* F = (FeedForwardLayer*)L;
@@ -2213,14 +2219,15 @@ static int begin_call(Net* n, const uint32_t* lens, uint32_t B, uint32_t S, cons
   }
   int S_alloc = (int)S, Sc = (int)S;
   for (const WaveletLayer* W : wl) {
-    Sc = T ? wavelet_rows(Sc - T, W->L) + T : wavelet_rows(Sc, W->L);
+    Sc = compressed_rows(W, Sc, T);
     if (T && Sc - T < 1) return fail(ERR_ARG, "%d target rows leave no input rows to compress", T);
     S_alloc = std::max(S_alloc, Sc);
   }
   if (mc != UINT32_MAX && (uint32_t)Sc > mc) return fail(ERR_ARG, "sequence %d exceeds max context %u", Sc, mc);
   Spec sz = sp;
   sz.S = S_alloc;
-  sz.S_out = wl.empty() ? 0 : Sc;
+  sz.S_first = wl.empty() ? 0 : (int)S;
+  sz.T = T;
   TRY(prepare(n, sz));
   if (sp.mode == MODE_PREFILL) TRY(alloc_caches(n, B));
   const size_t rows = (size_t)B * S;

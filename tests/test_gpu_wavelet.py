@@ -138,3 +138,30 @@ def test_wavelet_embedding_init_matches_oracle(vocab, src):
         g.init_embedding_wavelet(0, 7, 2048 if dim == 16 else 512)  # decomposes to 64 or 16 values
     g.close()
     o.close()
+
+
+def test_products_between_two_wavelet_layers():
+    """256 rows become 129 and then 66: the products between the two
+    compressions run at a row count that is neither the call's nor the
+    result's, with a split workspace of their own (rows of the middle length
+    take 96 tiles split 5 ways, 31 MB; 256 rows 128 tiles, 17 MB)."""
+    d, F = 512, 2048
+    r = np.random.default_rng(9)
+    x = r.standard_normal((1, 256, d)) + 1j * r.standard_normal((1, 256, d))
+
+    def build():
+        net = ra.Network(0)
+        net.add_discrete_wavelet(d, 1, 2)
+        net.add_feed_forward(d, F)
+        net.add_discrete_wavelet(d, 1, 2)
+        net.init_seeded(4)
+        return net
+
+    with build() as net:
+        y = net.forward_layers(0, 3, x, forward_only=False)
+    with build() as net:  # the same layers one at a time
+        h = net.forward_layers(0, 1, x, forward_only=False)
+        assert h.shape[1] == 129
+        want = net.forward_layers(2, 3, net.forward_layers(1, 2, h, forward_only=False), forward_only=False)
+    assert y.shape == want.shape == (1, 66, d)
+    assert np.array_equal(y, want)
