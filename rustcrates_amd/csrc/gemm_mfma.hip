@@ -256,8 +256,8 @@ __global__ __launch_bounds__(GNT, 6) void k_zgemm_mfma(const void* __restrict__ 
     __syncthreads();
     if constexpr (TA::real)
       if (bt.zero_row && m0 == 0 && tid < GBN && n0 + tid < N) {
-        if (bad[0][tid]) bt.zero_row[n0 + tid].x = NAN;
-        if (bad[1][tid]) bt.zero_row[n0 + tid].y = NAN;
+        // no MFMA forms this row, so the 0 * (infinity or NaN) they would meet shows here too
+        if (bad[0][tid] || bad[1][tid]) bt.zero_row[n0 + tid] = make_double2(NAN, NAN);
       }
 #pragma unroll
     for (int t = 0; t < GMT; ++t)

@@ -138,3 +138,25 @@ def test_second_backward_reads_the_updated_weights():
     z = x @ n1 + nb
     dh = oracle.linear_backward_c(gelu(z), gr, n2)[2]
     assert far(dx, oracle.dense_backward(x, z, dh, mask, n1)[2]) < TOL
+
+
+@pytest.mark.parametrize("bad", [complex(np.inf, 1.0), complex(0.5, -np.inf), complex(np.nan, 1.0), complex(1.0, np.nan)])
+def test_a_zero_gradient_row_meets_non_finite_head_weights(bad):
+    """The rows without a target have a zero gradient; times a weight that is
+    not finite, each of the four real products' sums is NaN."""
+    V, d, B, S, T = 90, 6, 2, 10, 3
+    r = np.random.default_rng(2)
+    table, w = c(r, V, d), 0.2 * c(r, d, V)
+    w[2, 71] = bad
+    ids, targets = r.integers(2, V, (B, S)).astype(np.uint32), r.integers(2, V, (B, T)).astype(np.uint32)
+    with ra.Network(0) as net:
+        net.add_embedding(V, d, table)
+        net.add_linear(d, V, w, np.zeros(V, np.complex128))
+        net.add_softmax(ra.TRAINING)
+        net.predict(ids, forward_only=False, want_output=False)
+        dx = net.backward_head(targets, update=False)
+    zero = np.ones(S, bool)
+    zero[S - T - 1:S - 1] = False  # the rows that predict a target
+    rest = [j for j in range(d) if j != 2]
+    assert np.isnan(dx[:, zero, 2].real).all() and np.isnan(dx[:, zero, 2].imag).all()
+    assert not dx[:, zero][:, :, rest].any()
