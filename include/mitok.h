@@ -326,6 +326,13 @@ int mitok_set_graph_mode(mitok_network* net, int direct_launch);
  * No counterpart in the reference (a scheduling choice; results agree to the
  * parity tolerance). */
 int mitok_set_decode_plan(mitok_network* net, int plan);
+/* Whether a stateless predict keeps each FeedForward's and attention layer's
+ * forward products (16 bytes of a row times 2 hidden, or 3 width) for
+ * backward.  1 (default): yes, where the device has room; they give way to any
+ * other allocation of the network, and a pass that needs as much as once had
+ * to give way keeps none (this call forgets that).  0: backward forms them
+ * again.  No counterpart in the reference; the results are the same bits. */
+int mitok_set_product_saving(mitok_network* net, int keep);
 /* Per-operation profile of the resident decode loop (plan 2).  enable = 1:
  * later launches record block 0's clock after every grid barrier.  Then, if
  * nops is not NULL, reports the last launch's operations (at most max_ops):

@@ -77,6 +77,7 @@ SIGNATURES = {
     "mitok_device_synchronize": (_i32, [_i32]),
     "mitok_set_graph_mode": (_i32, [_P, _i32]),
     "mitok_set_decode_plan": (_i32, [_P, _i32]),
+    "mitok_set_product_saving": (_i32, [_P, _i32]),
     "mitok_resident_exchange": (_i32, [_P, _i32, C.POINTER(_i32)]),
     "mitok_resident_profile": (_i32, [_P, _i32, _i32, C.POINTER(_i32), C.POINTER(_i32), C.POINTER(C.c_double)]),
 }
@@ -558,6 +559,11 @@ class Network:
 
     def set_graph_mode(self, direct_launch: bool):
         _check(self._lib.mitok_set_graph_mode(self._h, int(direct_launch)))
+
+    def set_product_saving(self, keep: bool):
+        """Whether a stateless predict keeps its FeedForward and attention
+        products for backward (the default) or backward forms them again."""
+        _check(self._lib.mitok_set_product_saving(self._h, int(keep)))
 
     def resident_profile(self, enable: bool = True):
         """Enables per-operation timing of the resident decode loop and returns

@@ -398,12 +398,17 @@ struct mitok_network {
   std::vector<std::unique_ptr<mitok::DevBuf>> tr_in, tr_cat;
   std::vector<char> tr_real;  // whether a layer's input rows had zero imaginary parts
   // the forward products backward reads: a FeedForward's pre-activation and
-  // hidden rows, an attention layer's q rows and its k and v rows.  tr_saved:
-  // the buffers are there (they are left out, and backward forms the products
-  // again, where the device has no room); tr_fresh: they hold the last
-  // stateless pass's values under the weights as they are
+  // hidden rows, an attention layer's q rows and its k and v rows.  They are
+  // the one thing here that can be done without (backward then forms the
+  // products again), so they give way to any other allocation the device has
+  // no room for.  tr_saved: the buffers are there for the last stateless pass;
+  // tr_fresh: they hold its values under the weights as they are; sv_limit:
+  // the bytes that once had to give way (later passes keep less or nothing,
+  // instead of allocating and freeing them each time)
   std::vector<std::unique_ptr<mitok::DevBuf>> sv_a, sv_b;
   bool tr_saved = false, tr_fresh = false;
+  size_t sv_limit = SIZE_MAX;
+  int keep_saved = 1;  // mitok_set_product_saving
   mitok::DevBuf tr_g, tr_xh, tr_dw, tr_db, tr_ga, tr_gb, tr_tgt, tr_norm;
   mitok::DevBuf tr_z, tr_h, tr_g1, tr_dh, tr_qkv, tr_dqkv, tr_A, tr_dA, tr_pg, tr_eid, tr_est, tr_eocc, tr_bsum;
   mitok::DevBuf ce_buf;  // mitok_cross_entropy_loss: targets, lengths, per-sequence losses, the result
@@ -426,9 +431,33 @@ static void drop_graph(Net* n) {
   n->graph = nullptr;
 }
 
+// Gives up the saved forward products; the bytes they held.
+static size_t drop_saved(Net* n) {
+  size_t held = 0;
+  for (auto* v : {&n->sv_a, &n->sv_b})
+    for (auto& b : *v) {
+      held += b->bytes;
+      b->release();
+    }
+  n->tr_saved = n->tr_fresh = false;
+  return held;
+}
+
+// Room for `bytes`, at the cost of the saved forward products if need be.  Not
+// between a pass's use of them and its end: no pass allocates once enqueued.
+static int alloc(Net* n, DevBuf& b, size_t bytes, bool* grew = nullptr) {
+  int rc = b.reserve(bytes, grew);
+  if (rc != ERR_NOMEM) return rc;
+  const size_t held = drop_saved(n);
+  if (!held) return rc;
+  rc = b.reserve(bytes, grew);
+  if (!rc) n->sv_limit = std::min(n->sv_limit, held);
+  return rc;
+}
+
 static int reserve(Net* n, DevBuf& b, size_t bytes) {
   bool grew = false;
-  TRY(b.reserve(bytes, &grew));
+  TRY(alloc(n, b, bytes, &grew));
   if (grew) {
     n->ws_generation++;
     drop_graph(n);
@@ -571,25 +600,33 @@ static bool is_vocab_linear(const Net* n, uint32_t li) {
 // a stateless pass of the whole stack is what backward may differentiate
 static bool keeps(const Spec& sp) { return sp.mode == MODE_STATELESS && !sp.hidden; }
 
-// Gives up the saved forward products: backward then forms them again.
-static void drop_saved(Net* n) {
-  for (auto* v : {&n->sv_a, &n->sv_b})
-    for (auto& b : *v) b->release();
-  n->tr_saved = n->tr_fresh = false;
-}
-
-// Room for the forward products of `rows` rows (at most) that backward reads
-static int reserve_saved(Net* n, const Spec& sp, size_t rows) {
+// Room for what a stateless pass leaves backward besides the layers' inputs:
+// the forward products of at most `rows` rows, or, where they are not kept,
+// the one scratch the pass then needs.  The last allocations before the pass
+// is enqueued.
+static int keep_products(Net* n, const Spec& sp, size_t rows) {
   for (auto* v : {&n->sv_a, &n->sv_b})
     while (v->size() < n->layers.size()) v->push_back(std::make_unique<DevBuf>());
-  for (uint32_t li = sp.first; li < sp.last; ++li) {
-    const Layer* L = n->layers[li].get();
-    const size_t a = L->kind == K_FEED_FORWARD ? ((const FeedForwardLayer*)L)->hidden : L->d_in;
-    if (L->kind != K_FEED_FORWARD && L->kind != K_SELF_ATTENTION) continue;
-    TRY(reserve(n, *n->sv_a[li], rows * a * sizeof(double2)));  // Z | q rows
-    TRY(reserve(n, *n->sv_b[li], rows * (L->kind == K_FEED_FORWARD ? a : 2 * a) * sizeof(double2)));  // H | k, v
-  }
-  return OK;
+  size_t total = 0;
+  const auto each = [&](auto use) -> int {
+    for (uint32_t li = sp.first; li < sp.last; ++li) {
+      const Layer* L = n->layers[li].get();
+      const bool ffn = L->kind == K_FEED_FORWARD;
+      if (!ffn && L->kind != K_SELF_ATTENTION) continue;
+      const size_t a = rows * (ffn ? ((const FeedForwardLayer*)L)->hidden : L->d_in) * sizeof(double2);
+      TRY(use(*n->sv_a[li], a));                // Z | q rows
+      TRY(use(*n->sv_b[li], ffn ? a : 2 * a));  // H | k and v rows
+    }
+    return OK;
+  };
+  (void)each([&](DevBuf&, size_t bytes) { return total += bytes, OK; });
+  // no graph holds them
+  n->tr_fresh = false;
+  n->tr_saved = n->keep_saved && total < n->sv_limit && each([](DevBuf& b, size_t bytes) { return b.reserve(bytes); }) == OK;
+  if (n->tr_saved) return OK;
+  drop_saved(n);
+  const Dims dm = net_dims(n);
+  return dm.hmax ? reserve(n, n->kv_scratch, 2 * rows * dm.dsa * sizeof(double2)) : OK;
 }
 
 // rows per sequence that a wavelet layer of a prompt or stateless pass leaves
@@ -665,14 +702,6 @@ static int prepare(Net* n, const Spec& sp) {
   if (n->pos_off) TRY(reserve(n, n->pos_off_d, (size_t)sp.B * sizeof(int)));
   TRY(reserve(n, n->ones_d, std::max<size_t>(rows, sp.B) * sizeof(uint32_t)));
   TRY(reserve(n, n->dec_ids_d, (size_t)sp.B * sizeof(uint32_t)));
-  if (keeps(sp)) {
-    n->tr_fresh = false;
-    n->tr_saved = reserve_saved(n, sp, rows) == OK;
-    if (!n->tr_saved) {  // no room: the pass itself needs only this
-      drop_saved(n);
-      if (dm.hmax) TRY(reserve(n, n->kv_scratch, 2 * rows * dm.dsa * c16));
-    }
-  }
   return OK;
 }
 
@@ -2101,7 +2130,7 @@ int mitok_init_embedding_wavelet(mitok_network* n, uint32_t layer, uint64_t seed
     return fail(ERR_ARG, "a %u-value draw decomposes to %d values, the layer's dim is %u", src_dim, dim, E->d_out);
   TRY(set_device(n));
   DevBuf kern;
-  TRY(kern.reserve(64 * sizeof(double2)));
+  TRY(alloc(n, kern, 64 * sizeof(double2)));
   const int rc = embedding_wavelet_init(n->stream, E->table.as<double2>(), (int)E->vocab, dim, (int)src_dim,
                                         stream_key(seed, stream_id(layer, 0xFFF)), kern.as<double2>(), 64);
   if (rc == ERR_HIP) return fail(ERR_HIP, "embedding wavelet init: %s", hipGetErrorString(hipGetLastError()));
@@ -2380,6 +2409,11 @@ static int predict_impl(mitok_network* n, const uint32_t* ids, const uint32_t* l
   TRY(upload(n, n->ids_d, padded.data(), rows * sizeof(uint32_t)));
   sp.ids = n->ids_d.as<uint32_t>();
   const uint32_t V = n->layers[n->layers.size() - 2]->d_out;
+  if (keeps(sp)) {
+    int widest = (int)S;  // rows per sequence at most, through the compressions
+    for (const auto& W : n->wstages) widest = std::max(widest, W->S2);
+    TRY(keep_products(n, sp, (size_t)B * widest));
+  }
   sp.out_re = n->logits_re.as<double>();
   sp.out_prob = n->probs.as<double>();
   TRY(enqueue_step(n, sp));
@@ -2439,7 +2473,7 @@ int mitok_cross_entropy_loss(mitok_network* n, const uint32_t* targets, const ui
   }
   TRY(set_device(n));
   const size_t tb = ((size_t)B * T + B) * sizeof(uint32_t), tb8 = (tb + 7) & ~(size_t)7;
-  TRY(n->ce_buf.reserve(tb8 + ((size_t)B + 2) * sizeof(double)));  // no graph holds it
+  TRY(alloc(n, n->ce_buf, tb8 + ((size_t)B + 2) * sizeof(double)));  // no graph holds it
   char* base = (char*)n->ce_buf.p;
   uint32_t* tgt_d = (uint32_t*)base;
   uint32_t* tlen_d = tgt_d + (size_t)B * T;
@@ -2511,8 +2545,8 @@ static int forward_layers_impl(Net* n, uint32_t first, uint32_t last, const doub
     sp.in = (const double2*)in;
     sp.out_hidden = (double2*)out;
   } else {
-    TRY(xin.reserve(rows * din * sizeof(double2)));
-    TRY(xout.reserve(orows * dout * sizeof(double2)));
+    TRY(alloc(n, xin, rows * din * sizeof(double2)));
+    TRY(alloc(n, xout, orows * dout * sizeof(double2)));
     HIP_TRY(hipMemcpyAsync(xin.p, in, rows * din * sizeof(double2), hipMemcpyHostToDevice, n->stream));
     sp.in = xin.as<double2>();
     sp.out_hidden = xout.as<double2>();
@@ -2865,15 +2899,16 @@ int mitok_decode_step(mitok_network* n, const uint32_t* ids, uint32_t B, uint32_
 
 // the AdamW moments of a weight (nw) and its bias (nb), allocated and zeroed
 // at the first update; nb = 0: a lone array's pair (mw, vw) only
-static int ensure_moments(hipStream_t st, size_t nw, size_t nb, DevBuf& mw, DevBuf& vw, DevBuf& mb, DevBuf& vb) {
+static int ensure_moments(Net* n, size_t nw, size_t nb, DevBuf& mw, DevBuf& vw, DevBuf& mb, DevBuf& vb) {
   if (mw.p && vw.p && (!nb || (mb.p && vb.p))) return OK;
-  TRY(mw.reserve(nw * sizeof(double2)));
-  TRY(vw.reserve(nw * sizeof(double2)));
+  hipStream_t st = n->stream;
+  TRY(alloc(n, mw, nw * sizeof(double2)));
+  TRY(alloc(n, vw, nw * sizeof(double2)));
   fill_const(st, mw.as<double2>(), nw, make_double2(0.0, 0.0));
   fill_const(st, vw.as<double2>(), nw, make_double2(0.0, 0.0));
   if (!nb) return OK;
-  TRY(mb.reserve(nb * sizeof(double2)));
-  TRY(vb.reserve(nb * sizeof(double2)));
+  TRY(alloc(n, mb, nb * sizeof(double2)));
+  TRY(alloc(n, vb, nb * sizeof(double2)));
   fill_const(st, mb.as<double2>(), nb, make_double2(0.0, 0.0));
   fill_const(st, vb.as<double2>(), nb, make_double2(0.0, 0.0));
   return OK;
@@ -3115,31 +3150,30 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
     }
     TRY(reserve(n, n->sync_ws, ws));
     if (update_params) {  // AdamW moments, zeroed at a layer's first update
-      TRY(ensure_moments(st, (size_t)d * V, V, Ln->mw, Ln->vw, Ln->mb, Ln->vb));
+      TRY(ensure_moments(n, (size_t)d * V, V, Ln->mw, Ln->vw, Ln->mb, Ln->vb));
       for (uint32_t li = stop; li < li_top; ++li) {
         Layer* L = n->layers[li].get();
         if (L->kind == K_LINEAR) {
           auto* H = (LinearLayer*)L;
-          TRY(ensure_moments(st, (size_t)H->d_in * H->d_out, H->d_out, H->mw, H->vw, H->mb, H->vb));
+          TRY(ensure_moments(n, (size_t)H->d_in * H->d_out, H->d_out, H->mw, H->vw, H->mb, H->vb));
         } else if (L->kind == K_FEED_FORWARD) {
           auto* F = (FeedForwardLayer*)L;
-          TRY(ensure_moments(st, (size_t)F->hidden * F->d_out, F->d_out, F->mw2, F->vw2, F->mb2, F->vb2));
-          TRY(ensure_moments(st, (size_t)F->d_in * F->hidden, F->hidden, F->mw1, F->vw1, F->mb1, F->vb1));
+          TRY(ensure_moments(n, (size_t)F->hidden * F->d_out, F->d_out, F->mw2, F->vw2, F->mb2, F->vb2));
+          TRY(ensure_moments(n, (size_t)F->d_in * F->hidden, F->hidden, F->mw1, F->vw1, F->mb1, F->vb1));
         } else if (L->kind == K_SELF_ATTENTION) {
           auto* A = (SelfAttentionLayer*)L;
-          TRY(ensure_moments(st, (size_t)3 * A->d_in * A->d_in, A->d_in, A->mw, A->vw, A->mg, A->vg));
-          TRY(ensure_moments(st, A->d_in, 0, A->mbt, A->vbt, A->mbt, A->vbt));
+          TRY(ensure_moments(n, (size_t)3 * A->d_in * A->d_in, A->d_in, A->mw, A->vw, A->mg, A->vg));
+          TRY(ensure_moments(n, A->d_in, 0, A->mbt, A->vbt, A->mbt, A->vbt));
         }
       }
     }
     return OK;
   };
-  int rc = size_all();
-  if (rc == ERR_NOMEM && n->tr_saved) {  // the forward pass's saved products give way
-    drop_saved(n);
-    rc = size_all();
-  }
-  if (rc) return rc;
+  bool had;
+  do {
+    had = n->tr_saved;
+    TRY(size_all());
+  } while (had != n->tr_saved);  // the saved products gave way meanwhile
   const bool fresh = n->tr_saved && n->tr_fresh;  // the saved forward products are of the weights as they are
   const Sync sy = sync_of(n);
   uint32_t* err = n->err_d.as<uint32_t>();
@@ -3472,8 +3506,8 @@ int mitok_greedy_decoding(mitok_network* n, const double* logits, uint32_t rows,
   if (!n || !logits || !out_ids || !rows || !V) return fail(ERR_ARG, "bad arguments");
   TRY(set_device(n));
   DevBuf lg, ids;
-  TRY(lg.reserve((size_t)rows * V * sizeof(double)));
-  TRY(ids.reserve((size_t)rows * sizeof(uint32_t)));
+  TRY(alloc(n, lg, (size_t)rows * V * sizeof(double)));
+  TRY(alloc(n, ids, (size_t)rows * sizeof(uint32_t)));
   HIP_TRY(hipMemcpyAsync(lg.p, logits, (size_t)rows * V * sizeof(double), hipMemcpyHostToDevice, n->stream));
   argmax_rows(n->stream, lg.as<double>(), rows, V, ids.as<uint32_t>(), n->err_d.as<uint32_t>());
   HIP_TRY(hipMemcpyAsync(out_ids, ids.p, rows * sizeof(uint32_t), hipMemcpyDeviceToHost, n->stream));
@@ -3544,6 +3578,13 @@ int mitok_device_synchronize(int device) {
 int mitok_set_graph_mode(mitok_network* n, int direct_launch) {
   if (!n) return fail(ERR_ARG, "null network");
   n->direct_launch = direct_launch;
+  return OK;
+}
+
+int mitok_set_product_saving(mitok_network* n, int keep) {
+  if (!n) return fail(ERR_ARG, "null network");
+  n->keep_saved = keep ? 1 : 0;
+  n->sv_limit = SIZE_MAX;
   return OK;
 }
 

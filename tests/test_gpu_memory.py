@@ -48,3 +48,49 @@ def test_a_refused_allocation_leaves_no_error_behind():
         ask_for_too_much(net)
         got, _ = net.predict(ids, lens=lens, forward_only=False)
     assert np.array_equal(got, want)
+
+
+def free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL("libamdhip64.so.7").hipMemGetInfo(C.byref(free), C.byref(total)) == 0  # the library's runtime
+    return free.value
+
+
+def step(net, ids, lens, targets, before_backward=lambda: None):
+    """One training step and a second backward under the new weights."""
+    P, _ = net.predict(ids, lens=lens, forward_only=False)
+    before_backward()
+    g1 = net.backward(targets, layers=net.num_layers - 1, update=True, learning_rate=0.05, time_step=1)
+    g2 = net.backward(targets, layers=4, update=False)
+    return [P, g1, g2, net.get_tensor(2, 0, 16 * 16), net.get_tensor(3, 0, 16 * 48), net.get_tensor(4, 0, 16 * 70)]
+
+
+def same(a, b):
+    return all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def test_backward_forms_products_that_were_not_kept():
+    """Kept products, none kept, and kept ones given up before backward: the
+    same kernels on the same rows, so the same bits."""
+    runs = []
+    for keep, give_up in ((True, False), (False, False), (True, True)):
+        net, ids, lens, targets = training_net()
+        with net:
+            net.set_product_saving(keep)
+            runs.append(step(net, ids, lens, targets, (lambda: ask_for_too_much(net)) if give_up else lambda: None))
+    assert np.abs(runs[0][1]).max() > 0 and not np.array_equal(runs[0][1], runs[0][2])
+    assert same(runs[0], runs[1]) and same(runs[0], runs[2])
+
+
+def test_kept_products_give_way_to_another_allocation():
+    net, ids, lens, targets = training_net(d=64, F=2048, S=400)
+    held = ids.size * 16 * (2 * 2048 + 3 * 64)
+    with net:
+        P, _ = net.predict(ids, lens=lens, forward_only=False)
+        before = free_bytes()
+        ask_for_too_much(net)
+        assert free_bytes() >= before + held // 2
+        loss = net.cross_entropy_loss(targets)
+        assert np.isfinite(loss.real)
+        after, _ = net.predict(ids, lens=lens, forward_only=False)  # nothing took their place: kept again
+        assert np.array_equal(after, P) and free_bytes() < before + held // 2
