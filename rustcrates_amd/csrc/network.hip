@@ -3175,6 +3175,7 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
     TRY(size_all());
   } while (had != n->tr_saved);  // the saved products gave way meanwhile
   const bool fresh = n->tr_saved && n->tr_fresh;  // the saved forward products are of the weights as they are
+  if (update_params) n->tr_fresh = false;         // from the first update on they are not, however the walk ends
   const Sync sy = sync_of(n);
   uint32_t* err = n->err_d.as<uint32_t>();
   long rows_c = rows;  // the current layer's rows (a wavelet layer changes them below it)
@@ -3420,10 +3421,7 @@ static int backward_impl(Net* n, const uint32_t* targets, const uint32_t* tlens,
       default: break;
     }
   }
-  if (update_params) {
-    drop_graph(n);  // the weights changed under any captured step
-    n->tr_fresh = false;
-  }
+  if (update_params) drop_graph(n);  // the weights changed under any captured step
   if (out_grad_input) {
     const int dlow = (int)n->layers[stop]->d_in;
     HIP_TRY(hipMemcpyAsync(out_grad_input, gcur, (size_t)rows_c * dlow * c16, hipMemcpyDeviceToHost, st));
