@@ -407,9 +407,11 @@ int attention_decode_split(hipStream_t st, const Attn& a, const double2* q, long
 // [qr | qi], and v_mfma_f64_16x16x4_f64 forms 16x16 score tiles.  Scores get
 // the scale and Re(bias_pos[r][c]); keys c > r get -1e12
 // (masked_attention_head.rs:189-203).  The softmax runs online (running row
-// max m and sum l, the partial output rescaled by e^(m_old - m_new)); masked keys contribute exactly 0.  P goes through LDS to become the
-// A operand of the P.V MFMAs (values staged in LDS).  Key groups are merged at
-// the end like key chunks; out = acc / l; pad rows give 0.
+// max m and sum l, the partial output rescaled by e^(m_old - m_new)); masked
+// keys contribute exactly 0, or NaN where their values are not finite.  P goes
+// through LDS to become the A operand of the P.V MFMAs (values staged in LDS).
+// Key groups are merged at the end like key chunks; out = acc / l; pad rows
+// give 0.
 // D[i][j] of a 16x16 tile sits at lane j + 16*(i%4), element i/4.
 //
 // Bound by the matrix cores once they are kept busy: the next tile's keys,
@@ -570,6 +572,29 @@ __global__ __launch_bounds__(64 * NW * KG, DH <= 64 ? 2 : 1) void k_attention_pr
       }
     }
     __builtin_amdgcn_wave_barrier();
+  }
+  // A masked key weighs 0, and 0 * (infinity or NaN) is NaN: row r's output is
+  // NaN in the columns where a key past r is not finite.  The tiles past a
+  // wave's rows are skipped above, so where the values' product has seen such
+  // a value, each column's last one is looked for among all keys.
+  if (a.v_bad && *a.v_bad) {
+    __shared__ int last[2][DH];
+    for (int t = tid; t < 2 * DH; t += NTH) last[t / DH][t % DH] = -1;
+    __syncthreads();
+    for (int idx = tid; idx < T * dh; idx += NTH) {
+      const double2 vv = Vc[idx];
+      const int c = idx / dh, e = idx - c * dh;
+      if (!isfinite(vv.x)) atomicMax(&last[0][e], c);
+      if (!isfinite(vv.y)) atomicMax(&last[1][e], c);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int t = 0; t < ET; ++t) {
+        if (last[0][16 * t + i] > r0 + 4 * e + kq) o_re[t][e] = NAN;
+        if (last[1][16 * t + i] > r0 + 4 * e + kq) o_im[t][e] = NAN;
+      }
   }
   if constexpr (KG > 1) {
     // key group 0 of each row wave takes the others' (max, sum, output) in

@@ -90,6 +90,7 @@ struct Epi {
   uint32_t* err = nullptr;
   // EPI_QKV: row m = b * S + s
   int d = 0, dh = 0, heads = 0, S = 1;
+  uint32_t* v_bad = nullptr;  // QKV: set to 1 where a value row is not finite
   double2* kc = nullptr;  // [B][heads][ctx][dh]
   double2* vc = nullptr;
   int ctx = 0;
@@ -140,6 +141,7 @@ struct Attn {
   const double* bias_re = nullptr;  // [H][mc][mc] Re(bias_pos)
   int mc = 0;
   const uint32_t* row_mask = nullptr;  // [B*S]
+  const uint32_t* v_bad = nullptr;     // attention_prefill: not 0 where some value may not be finite (null: never)
   double2* out = nullptr;              // [B*S][ldo], head h at column h*dh
   long ldo = 0;
   int B = 0, S = 0, H = 0, dh = 0;

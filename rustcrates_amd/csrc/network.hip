@@ -472,12 +472,14 @@ static int upload(Net* n, DevBuf& b, const void* src, size_t bytes) {
 }
 
 static int check_err_word(Net* n) {
-  uint32_t e = 0;
-  HIP_TRY(hipMemcpyAsync(&e, n->err_d.p, sizeof e, hipMemcpyDeviceToHost, n->stream));
+  uint32_t w[2] = {0, 0};  // the error word, and whether a value row was not finite (Epi::v_bad)
+  HIP_TRY(hipMemcpyAsync(w, n->err_d.p, sizeof w, hipMemcpyDeviceToHost, n->stream));
   HIP_TRY(hipStreamSynchronize(n->stream));
+  if (!w[0] && !w[1]) return OK;
+  fill_u32(n->stream, n->err_d.as<uint32_t>(), 2, 0);
+  HIP_TRY(hipStreamSynchronize(n->stream));
+  const uint32_t e = w[0];
   if (!e) return OK;
-  fill_u32(n->stream, n->err_d.as<uint32_t>(), 1, 0);
-  HIP_TRY(hipStreamSynchronize(n->stream));
   if (e & EB_BAD_TOKEN) return fail(ERR_ARG, "No token embedding found: token id >= vocab (embedding_layer.rs:305)");
   if (e & EB_GELU_NAN) return fail(ERR_NAN, "NaN detected in tanh(f(z)) (activation.rs:207-209)");
   if (e & EB_FFN_NONFINITE) return fail(ERR_NAN, "output ffn dense: The value is Not Valid (transformer_network.rs:408)");
@@ -835,6 +837,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         e.heads = H;
         e.S = S;
         e.err = err;
+        e.v_bad = err + 1;
         Attn a;
         a.q = q;
         a.ldq = d;
@@ -870,6 +873,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         a.bias_re = A->bias_re.as<double>();
         a.mc = A->max_ctx;
         a.row_mask = mask;
+        a.v_bad = err + 1;
         a.out = cat;
         a.ldo = d;
         a.B = B;
@@ -1873,10 +1877,10 @@ int mitok_network_create(int device, mitok_network** out) {
   if (!rc && hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking) != hipSuccess)
     rc = fail(ERR_HIP, "hipStreamCreate failed");
   if (!rc) rc = noalloc_scratch(device, &n->scratch);
-  if (!rc) rc = n->err_d.reserve(sizeof(uint32_t));
+  if (!rc) rc = n->err_d.reserve(2 * sizeof(uint32_t));
   if (!rc) rc = n->sync_cnt.reserve((size_t)SYNC_COUNTERS * sizeof(uint32_t));
   if (!rc) {
-    fill_u32(n->stream, n->err_d.as<uint32_t>(), 1, 0);
+    fill_u32(n->stream, n->err_d.as<uint32_t>(), 2, 0);
     fill_u32(n->stream, n->sync_cnt.as<uint32_t>(), SYNC_COUNTERS, 0);
     if (hipStreamSynchronize(n->stream) != hipSuccess) rc = fail(ERR_HIP, "stream sync failed");
   }

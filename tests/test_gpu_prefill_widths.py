@@ -51,3 +51,30 @@ def test_prefill_attention_blocks(B, S, H, dh):
     want = t / np.sqrt((t * t).mean(-1, keepdims=True) + 1e-12)
     assert np.all(got.imag == 0)
     assert np.max(np.abs(got.real - want)) < 1e-12 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("B,S,H,dh,at", [(2, 100, 2, 16, 40), (1, 33, 1, 64, 32), (130, 40, 4, 20, 39), (1, 300, 2, 32, 299),
+                                         (40, 200, 5, 24, 130), (1, 70, 2, 128, 66)])
+def test_a_later_row_that_is_not_finite_reaches_the_earlier_ones(B, S, H, dh, at):
+    """A masked key has weight 0, and 0 times a value that is not finite is
+    NaN (utils/matrix.rs:356-380 sums over every key): the tiled kernel, which
+    skips masked tiles, against the one-row-per-block form."""
+    d = H * dh
+    r = np.random.default_rng(at)
+    c = lambda *s: r.standard_normal(s) + 1j * r.standard_normal(s)  # noqa: E731
+    wq, wk, wv = (c(H, d, dh) / np.sqrt(2 * d) for _ in range(3))
+    x = c(B, S, d)
+    x[0, at, 3] = complex(np.inf, 0.5)
+    mask = np.ones((B, S), np.uint32)
+    mask[:, 0] = 0  # a padded row stays 0
+    out = []
+    for plan in (1, 0):
+        with ra.Network(0) as net:
+            net.add_self_attention(H, d, S, 1e-12, wq, wk, wv, 0.3 * np.ones((H, S, S)))
+            net.set_decode_plan(plan)
+            out.append(net.forward_layers(0, 1, x, mask=mask, forward_only=False))
+    tiled, rows = out
+    assert np.array_equal(np.isnan(tiled), np.isnan(rows))
+    assert np.isnan(rows[0, 1:].real).all() and np.isfinite(rows[0, 0]).all() and np.isfinite(rows[1:]).all()
+    live = np.isfinite(rows)
+    assert np.max(np.abs(tiled[live] - rows[live])) < 1e-12 * np.max(np.abs(rows[live]))
