@@ -41,6 +41,13 @@ _HOST_FEATURE_NOTE = "'-packed-fp32-ops' is not a recognized feature"
 FILE_FLAGS = {"gemm_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               # the optimizer's arithmetic rounds every multiply and add, as Rust does
               "train.hip": ["-ffp-contract=off"],
+              # 4 and 8 rows: the constants of tanh's exponential and sine were held in registers
+              # across the resident loop and spilled others (51 VGPRs in the 8-row barrier form);
+              # formed where they are used, nothing spills.  us per step at width 512, prompts of
+              # 128, with / without: 8 rows 840 / 868 behind barriers, 721 / 724 polled, 4 rows 489 /
+              # 506 and 417 / 423.  One row behind barriers is slower with it (286 / 282), two equal
+              "resident_k4.hip": ["-mllvm", "-disable-machine-licm"],
+              "resident_k8.hip": ["-mllvm", "-disable-machine-licm"],
               # the wavelet embedding follows the reference's multiply and add order
               "wavelet_init.hip": ["-ffp-contract=off"]}
 
