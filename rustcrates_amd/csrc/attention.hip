@@ -420,8 +420,9 @@ int attention_decode_split(hipStream_t st, const Attn& a, const double2* q, long
 // built ones run the next wider with zeros.  MI355X, head dim 64, us, against
 // blocks of 128 rows that loaded each tile when it was needed: 48 heads of 1920
 // rows 1822 -> 1573, 768 of 256 765 -> 545, 256 of 128 74 -> 54, 64 of 256 117
-// -> 69, 36 of 173 80 -> 37.  What is left is the softmax: two exponentials per
-// 16 MFMAs in a wave that waits for each tile's scores.
+// -> 69, 36 of 173 80 -> 37 (blocks of 32 rows spill 6 of their 256 VGPRs).
+// What is left is the softmax: two exponentials per 16 MFMAs in a wave that
+// waits for each tile's scores.
 // ===========================================================================
 template <int DH, int NW, int KG>
 __global__ __launch_bounds__(64 * NW * KG, DH <= 64 ? 2 : 1) void k_attention_prefill(Attn a) {

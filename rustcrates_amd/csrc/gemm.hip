@@ -1165,7 +1165,9 @@ static SkinnyPlan plan_skinny(int M, int N, int K, bool part, bool argmax) {
     // 768 of K per block where that divides K and the grid still fills the
     // chip: K 768 in 512s leaves half the second block's waves idle and a
     // partial more for the consumer (64 rows at width 768, the layer products
-    // of a decode step together, with the real rows below: 106 -> 94 us)
+    // of a decode step together, with the real rows below: 106 -> 94 us).  K
+    // that 768 only pads less than 512 does (700, 1280) stays with 512: not
+    // measured
     r.nkw = K % 768 == 0 && (long)r.ncb * r.rt * (K / 768) >= 256 && K / 768 <= SKINNY_MAX_SPLIT ? 12 : 8;
     int P = cdiv_i(K, 64 * r.nkw);
     if (!part) {

@@ -29,9 +29,10 @@ namespace mitok {
 // result is what the four products give.
 //
 // Why this tile: a wave step is 64 cycles per MFMA, so the loop is bound by how
-// well loads and barriers hide behind it.  With 80 registers a wave and 32 KB
-// of LDS a block, three blocks (six waves per SIMD) share a CU and one's
-// barrier is covered by another's MFMAs; global loads go out two K steps
+// well loads and barriers hide behind it.  With 80 registers a wave (the real
+// QKV form and seven of backward's spill 1 to 3 more) and 32 KB of LDS a block,
+// three blocks (six waves per SIMD) share a CU and one's barrier is covered by
+// another's MFMAs; global loads go out two K steps
 // ahead into registers, fragments one 4-k step ahead.  Measured on MI355X
 // (TFLOP/s at 8, real A 4 flops per complex multiply-add), against 64x64 with
 // 4 waves of 32x32, K step 16, one step ahead:

@@ -308,7 +308,11 @@ __global__ __launch_bounds__(1024) void k_softmax_rows_wide(double* __restrict__
 }
 
 // 256 threads where 8 values each hold the row, else 1024 threads with the
-// fewest registers that do (52 values: 104 VGPRs of the 128 a 1024-thread block may use)
+// fewest registers that do.  52 values do not all fit the 128 VGPRs a
+// 1024-thread block may use (49 go to scratch), which still beats three passes
+// where there are rows enough (us at V 50280 against k_softmax_rows_wide: 256
+// rows 68 / 79, 1024 321 / 335, 4096 1233 / 1288, but 64 rows 53 / 49; at V
+// 36864 about equal: 50 / 58, 238 / 236, 946 / 896, 42 / 37)
 void softmax_rows(hipStream_t st, double* x, int rows, int S, int V, const uint32_t* row_mask, int mode) {
   if (V <= 256 * 8) hipLaunchKernelGGL((k_softmax_rows<256, 8>), dim3(rows), dim3(256), 0, st, x, S, V, row_mask, mode);
   else if (V <= 1024 * 8) hipLaunchKernelGGL((k_softmax_rows<1024, 8>), dim3(rows), dim3(1024), 0, st, x, S, V, row_mask, mode);

@@ -75,7 +75,8 @@ void linear_update(hipStream_t st, double2* W, const double2* dW, double2* mW, d
 // the Norm's backward per row of x (or Re(x + resid) + 0i); dx real rows, pg = dout * x_hat
 void norm_backward(hipStream_t st, const double2* x, const double2* resid, long rows, int n, double eps,
                    const double2* gamma, const double2* beta, const double2* dout, double2* dx, double2* pg);
-// out[j] = mult * sum over sequences b of the row sum of X[b][:][j] (rows in order, then sequences); ws [B][n]
+// out[j] = mult * sum over sequences b of the row sum of X[b][:][j] (four runs of rows, each in order, then the
+// sequences in order); ws [B][n]
 void colsum(hipStream_t st, const double2* X, int B, int S, int n, double mult, double2* ws, double2* out);
 // the same of packed real rows, sequence b's at [starts[b], starts[b + 1])
 void colsum_packed(hipStream_t st, const double* X, const int* starts, int B, int n, double2* ws, double2* out);

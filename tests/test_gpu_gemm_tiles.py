@@ -79,3 +79,25 @@ def test_real_rows_meet_infinities_and_nan_as_complex_ones_do(rows, k):
         assert np.array_equal(np.isnan(got), np.isnan(want))
         inf = np.isinf(want)
         assert inf.any() and np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], want[inf])
+
+
+@pytest.mark.parametrize("rows,d,V", [(70, 512, 9600), (130, 200, 6400), (65, 512, 64)])
+def test_greedy_ids_of_a_split_last_round(rows, d, V):
+    """The vocabulary product of more than 64 sequences forms each row's id in
+    its epilogue: with whole tiles and split ones in one launch (150 column
+    tiles of 2 row tiles, 100 of 3), and with every tile split."""
+    r = np.random.default_rng(V)
+    table = r.standard_normal((rows + 3, d)) + 1j * r.standard_normal((rows + 3, d))
+    w = r.standard_normal((d, V)) + 1j * r.standard_normal((d, V))
+    b = r.standard_normal(V) + 1j * r.standard_normal(V)
+    ids = np.arange(2, rows + 2, dtype=np.uint32)[:, None]
+    with ra.Network(0) as net:
+        net.add_embedding(rows + 3, d, table)
+        net.add_linear(d, V, w, b)
+        net.add_softmax(ra.PRODUCTION)
+        got, lg = net.generate(ids, lens=np.ones(rows, np.uint32), n_new=1, want_logits=True)
+    x = table[ids[:, 0]]
+    bound = (d + 4) * EPS * (np.abs(x) @ np.abs(w) + np.abs(b))
+    lg = np.asarray(lg).reshape(rows, V)
+    assert np.all(np.abs(lg - (x @ w + b).real) <= bound)
+    assert np.array_equal(np.asarray(got).reshape(rows), V - 1 - np.argmax(lg[:, ::-1], axis=1))  # the last of equal ones

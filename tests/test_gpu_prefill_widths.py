@@ -32,7 +32,8 @@ def heads_output(x, wq, wk, wv, bias, mask):
 
 # (B, S, H, dh): 32-row blocks with ragged ends, 64-row ones, 128-row ones; head dims between the built ones
 @pytest.mark.parametrize("B,S,H,dh", [(1, 1, 2, 16), (2, 33, 2, 24), (1, 97, 1, 64), (64, 65, 2, 16), (70, 30, 4, 20),
-                                      (130, 40, 4, 8), (40, 129, 5, 40), (2, 70, 2, 100), (1, 31, 1, 128)])
+                                      (130, 40, 4, 8), (40, 129, 5, 40), (2, 70, 2, 100), (1, 31, 1, 128),
+                                      (130, 40, 4, 20), (43, 150, 4, 32)])
 def test_prefill_attention_blocks(B, S, H, dh):
     d = H * dh
     r = np.random.default_rng(S * dh)
