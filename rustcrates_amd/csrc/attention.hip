@@ -578,7 +578,7 @@ __global__ __launch_bounds__(64 * NW * KG, DH <= 64 ? 2 : 1) void k_attention_pr
   // NaN in the columns where a key past r is not finite.  The tiles past a
   // wave's rows are skipped above, so where the values' product has seen such
   // a value, each column's last one is looked for among all keys.
-  if (a.v_bad && *a.v_bad) {
+  if (a.err && a.err[1]) {
     __shared__ int last[2][DH];
     for (int t = tid; t < 2 * DH; t += NTH) last[t / DH][t % DH] = -1;
     __syncthreads();

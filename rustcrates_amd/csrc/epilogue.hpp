@@ -53,7 +53,7 @@ __device__ __forceinline__ double apply_epi(const Epi& ep, int M, int N, int m, 
         break;
       }
       if constexpr (std::is_same<Acc, AccPlain>::value)
-        if (part == 2 && ep.v_bad && !(isfinite(v.x) && isfinite(v.y))) *ep.v_bad = 1u;
+        if (part == 2 && !(isfinite(v.x) && isfinite(v.y))) ep.err[1] = 1u;
       double2* dst = part == 1 ? ep.kc : ep.vc;
       Acc::st(dst + (((long)b * ep.heads + h) * ep.ctx + pos) * ep.dh + e, v);
       break;

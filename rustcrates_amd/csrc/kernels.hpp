@@ -87,10 +87,9 @@ struct Epi {
   const uint32_t* row_mask = nullptr;  // GELU: rows with mask 0 become 0
   double2* pre = nullptr;              // GELU: also pre[m][n] = v + bias, as backward reads it (ld ldo)
   int check_finite = 0;
-  uint32_t* err = nullptr;
+  uint32_t* err = nullptr;  // [2]: the error word; QKV: 1 where a value row is not finite
   // EPI_QKV: row m = b * S + s
   int d = 0, dh = 0, heads = 0, S = 1;
-  uint32_t* v_bad = nullptr;  // QKV: set to 1 where a value row is not finite
   double2* kc = nullptr;  // [B][heads][ctx][dh]
   double2* vc = nullptr;
   int ctx = 0;
@@ -141,14 +140,13 @@ struct Attn {
   const double* bias_re = nullptr;  // [H][mc][mc] Re(bias_pos)
   int mc = 0;
   const uint32_t* row_mask = nullptr;  // [B*S]
-  const uint32_t* v_bad = nullptr;     // attention_prefill: not 0 where some value may not be finite (null: never)
   double2* out = nullptr;              // [B*S][ldo], head h at column h*dh
   long ldo = 0;
   int B = 0, S = 0, H = 0, dh = 0;
   double scale = 1.0;
   double2* kc_w = nullptr;  // writable cache (attention_decode_split appends the new token)
   double2* vc_w = nullptr;
-  uint32_t* err = nullptr;
+  uint32_t* err = nullptr;  // as Epi's; null: every value is finite
 };
 // One query row per block (the general reference case, any T).
 void attention_rows(hipStream_t st, const Attn& a);

@@ -472,7 +472,7 @@ static int upload(Net* n, DevBuf& b, const void* src, size_t bytes) {
 }
 
 static int check_err_word(Net* n) {
-  uint32_t w[2] = {0, 0};  // the error word, and whether a value row was not finite (Epi::v_bad)
+  uint32_t w[2] = {0, 0};  // the error word, and whether a value row was not finite (EPI_QKV, attention_prefill)
   HIP_TRY(hipMemcpyAsync(w, n->err_d.p, sizeof w, hipMemcpyDeviceToHost, n->stream));
   HIP_TRY(hipStreamSynchronize(n->stream));
   if (!w[0] && !w[1]) return OK;
@@ -837,7 +837,6 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         e.heads = H;
         e.S = S;
         e.err = err;
-        e.v_bad = err + 1;
         Attn a;
         a.q = q;
         a.ldq = d;
@@ -873,7 +872,7 @@ static int enqueue_forward(Net* n, const Spec& sp) {
         a.bias_re = A->bias_re.as<double>();
         a.mc = A->max_ctx;
         a.row_mask = mask;
-        a.v_bad = err + 1;
+        a.err = err;
         a.out = cat;
         a.ldo = d;
         a.B = B;
